@@ -210,3 +210,38 @@ def test_host_emitters_follow_pixel_size_type(model, dtype):
         # a Float32 pixel size of the same nominal value rounds differently somewhere
         alt = mirror(model, box, params.T, crlb.T, llr, xc, yc, float(F32(psx)), float(F32(psy)))[:, :2]
         assert np.any(alt != want[:, :2])
+
+
+@pytest.mark.parametrize("df", [1, 2, 3, 4, 7, 45, 1019, 1020])
+def test_chi2_pvalue_at_the_edges_of_its_two_sums(hiplib, df):
+    """Either side of chi2 = df/2, where the power series hands over to the
+    finite sum, of chi2 = 74, where an odd df's erfc term ends, and the tails
+    where the sum stops early.  The CDF is a Float64 sum, rounded to Float32
+    once: p is within one Float32 step at 1."""
+    c = np.array([0.5 * df * f for f in (1e-3, 0.5, 0.999, 1.0, 1.001, 1.5, 2.0, 2.5, 4.0, 40.0)] +
+                 [73.9, 74.0, 74.1, 1e-6, 1e4, 1e30], dtype=F32)
+    got = np.array([hiplib.gmle_chi2_pvalue(float(x), df) for x in c], dtype=F32)
+    np.testing.assert_allclose(got, reference_pvalue(c, df), rtol=0, atol=np.spacing(F32(0.5)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1031])
+def test_epilogue_device_ragged_blocks(n):
+    """Batches that fill the last block, or one ROI of it; 3 and 32 px boxes."""
+    import torch
+    from gaussmle_amd.device import epilogue_device
+    rng = np.random.default_rng(n)
+    for model, box in ((2, 3), (1, 32)):
+        P = [4, 5, 6, 5][model]
+        params, crlb = (np.abs(rng.normal(5, 2, (n, P))).astype(F32) for _ in range(2))
+        llr = (-rng.chisquare(box * box - P, n) / 2).astype(F32)
+        xc, yc = (rng.integers(1, 2000, n).astype(np.int32) for _ in range(2))
+        d = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+        out = torch.full((n + 1, 10), -7.0, device="cuda")
+        epilogue_device(d(params), d(crlb), d(llr), 0.1, 0.107, model, box, d_xc=d(xc), d_yc=d(yc), out=out)
+        got = out.cpu().numpy()
+        want = mirror(model, box, params, crlb, llr, xc, yc, 0.1, 0.107)
+        for q in (0, 1, 2, 3, 5, 6, 7, 8, 9):
+            np.testing.assert_array_equal(got[:n, q], want[:, q], err_msg=f"field {q}")
+        np.testing.assert_allclose(got[:n, 4], want[:, 4], rtol=0, atol=np.spacing(F32(0.5)))
+        assert np.all(got[n] == -7.0)   # nothing past the last ROI
