@@ -13,7 +13,8 @@
 //     "The transformed rejection method for generating Poisson random
 //     variables", Insurance: Mathematics and Economics 12, 1993);
 //   normal: Box-Muller.
-// Arithmetic is Float64 (the generator is not a hot path).
+// Arithmetic is Float64.  The simulator kernel (gmle_sim.hip) decides most
+// Poisson draws in Float32 within guard bands and comes here for the rest.
 #pragma once
 
 #include <hip/hip_runtime.h>

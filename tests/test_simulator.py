@@ -130,6 +130,30 @@ def test_device_matches_oracle_ideal(model):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("box,n", [(3, 1), (3, 1501), (5, 64), (6, 700), (11, 130), (32, 37)])
+def test_device_counts_equal_the_float64_samplers(box, n):
+    """Flat ROIs (no emitter), whose expected count is the background itself:
+    every count equals the Float64 samplers' of the oracle, across both methods
+    and their seam at 10, counts drawn in Float64 above 1e6, backgrounds that
+    draw nothing, and batches that end inside a wave's list."""
+    import torch
+    rng = np.random.default_rng(box * 1000 + n)
+    bg = np.exp(rng.uniform(np.log(1e-3), np.log(3e4), n)).astype(np.float32)
+    special = np.array([10.0, np.nextafter(np.float32(10), np.float32(0)), 10.5, 9.5, 0.0, -1.0, np.nan, 1e-6, 999_999.0,
+                        1_000_001.0, 3e6, 12.0, 0.5], np.float32)
+    bg[::2] = special[np.arange(len(bg[::2])) % len(special)]
+    c = (box + 1) / 2
+    params = np.stack([np.full(n, c), np.full(n, c), np.zeros(n), bg], axis=1).astype(np.float32)
+    want, exp = refsim.simulate(GaussianXYNB(1.3), box, params, seed=n)
+    np.testing.assert_array_equal(exp, np.repeat(bg, box * box))
+    out = torch.full((n * box * box + 8,), -5.0, device="cuda")
+    gsim.simulate_device(GaussianXYNB(1.3), box, torch.from_numpy(params).cuda(), n, out=out)
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:-8], want)
+    assert np.all(got[-8:] == -5.0)
+
+
+@pytest.mark.gpu
 def test_device_matches_oracle_scmos_maps():
     import torch
     rng = np.random.default_rng(60)
