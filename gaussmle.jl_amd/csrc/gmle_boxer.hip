@@ -21,17 +21,18 @@
 //   order: by frame, then column-major pixel index (Julia's findall order).
 //
 // Kernels (all deterministic; no atomics):
-//   1. boxer_dog: one tile of 62 rows x 30 columns per block, staged through
-//      LDS with a halo of R + 1; each pass runs over register strips of 8
-//      outputs (one LDS read per input value and strip); writes D and, per
-//      tile column, a ballot word of the 3x3 maxima above minval (a necessary
-//      condition).
+//   1. boxer_detect: filters and finds the 3 x 3 maxima above minval (a
+//      necessary condition) in one sweep.  Writes one 64-bit word of candidates
+//      per column and word_rows rows.  D stays in LDS except around pixels
+//      above minval: where a step of a wave has one, its D is stored and its
+//      words are flagged.  (Anything not stored is at most minval and beats no
+//      candidate.)
 //   2. boxer_suppress: one candidate word per lane; a wave tests its lanes'
 //      candidates one at a time, reading each window with all 64 lanes;
-//      per-block survivor counts.
+//      survivors per block of words.
 //   3. boxer_scan: exclusive scan of the block counts; total detections.
-//   4. boxer_place: each survivor's rank from the scan -> corners and frame.
-//   5. boxer_cut: one wave per box copies its pixels.
+//   4. boxer_place: each survivor's rank from the scan -> corners and frame;
+//      then the block copies its boxes, one wave per box.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -45,16 +46,18 @@
 namespace gmle {
 namespace {
 
-constexpr int kDRows = 64;         // filtered region per tile: rows (the contiguous axis) ...
-constexpr int kDCols = 32;         // ... and columns, with a 1-pixel halo around the interior
-constexpr int kWordRows = kDRows - 2;   // 62 interior rows: one candidate word per tile column
-constexpr int kInnerCols = kDCols - 2;  // 30 interior columns
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kMaxRadius = 12;     // weights radius limit: sigma <= 4 px
-constexpr int kStrip = 8;          // outputs per thread along the filter axis
+constexpr int kStep = 8;           // columns per step of the sweep
+constexpr int kStrip = 8;          // rows per thread of the y pass
+constexpr int kRing = 16;          // columns of D in LDS, at least kStep + 2
+constexpr uint64_t kStored = 1ull << 63;   // candidate word: D of its rows is stored
+constexpr int kWordsPerThread = 4; // boxer_suppress / boxer_place, at most
 constexpr int kScanThreads = 1024;
-constexpr int kCutBlocks = 4096;
+constexpr int kTargetBlocks = 3 * 5 * 256;   // boxer_detect runs five blocks per CU
+constexpr int kMinSweep = 24;
+constexpr int64_t kManyWords = 1 << 19;
 
 struct BoxerArgs {
   const float* frames;   // (ny, nx, nf) column-major
@@ -66,11 +69,14 @@ struct BoxerArgs {
   float minval;
   int win;               // suppression radius r
   int box;
-  int wpc;               // candidate words per column: ceil(ny / 62)
+  int word_rows;         // rows per word
+  int wpc;               // words per column: ceil(ny / word_rows)
+  int sweep;             // columns per block of boxer_detect
   int64_t n_words;       // nf * nx * wpc
   int64_t max_boxes;
-  float* dog;            // (ny, nx, nf)
-  uint64_t* cand;        // (wpc, nx, nf); bit b of word w <-> row 62 w + b
+  int wpt;               // words per thread of suppress / place: 1, or kWordsPerThread for large stacks
+  float* dog;            // (ny, nx, nf), where the word is kStored
+  uint64_t* cand;        // (wpc, nx, nf); bit b of word w <-> row word_rows w + b
   uint64_t* keep;        // (wpc, nx, nf)
   int64_t* block_base;   // per suppress / place block
   int64_t* count;        // total detections
@@ -81,155 +87,191 @@ struct BoxerArgs {
   float* strength;       // D at the detection (may be null)
 };
 
-// LDS layout of a tile for radii up to RMAX.  Rows and columns are stored
-// with an offset of RMAX, so every strip reads the same 8 + 2 RMAX values
-// whatever the actual radius (the values beyond it are never used), and the
-// row stride is odd, so lanes reading one value per column hit different banks.
-template <int RMAX>
-struct TileLayout {
-  static constexpr int kRows = kDRows + 2 * RMAX;         // stored rows of `in`, `hs`, `hl`
-  static constexpr int kStride = kRows | 1;
-  static constexpr int kInCols = kDCols + 2 * RMAX;
-  static constexpr int kDStride = kDRows | 1;
-  static constexpr int kWeights = 2 * (kMaxRadius + 1);
-  static constexpr int kFloats = kWeights + kInCols * kStride + 2 * kDCols * kStride;
-  static constexpr int kStripLen = kStrip + 2 * RMAX;
-};
+// Rows per candidate word: four words and a halo of radius + 1 above and below
+// fit the 256 rows of a block.
+__host__ __device__ constexpr int word_rows_of(int rmax) { return rmax <= 6 ? 60 : 56; }
 
 // One Gaussian over a register strip: out[o] = w0 x[c+o] + sum_k w_k
-// (x[c+o-k] + x[c+o+k]), fma in increasing k, c = RMAX.  R is uniform.
-template <int RMAX>
-__device__ __forceinline__ void strip_filter(const float (&x)[kStrip + 2 * RMAX], const float* w, int R,
-                                             float (&out)[kStrip]) {
+// (x[c+o-k] + x[c+o+k]), fma in increasing k, c = RMAX.  The radius is FIXED,
+// or the uniform R where FIXED is 0.
+template <int RMAX, int FIXED, int N>
+__device__ __forceinline__ void strip_filter(const float (&x)[N + 2 * RMAX], const float* w, int R, float (&out)[N]) {
 #pragma clang fp contract(off)
   const float w0 = w[0];
 #pragma unroll
-  for (int o = 0; o < kStrip; ++o) out[o] = w0 * x[RMAX + o];
+  for (int o = 0; o < N; ++o) out[o] = w0 * x[RMAX + o];
 #pragma unroll
-  for (int k = 1; k <= RMAX; ++k) {
-    if (k <= R) {
+  for (int k = 1; k <= (FIXED ? FIXED : RMAX); ++k) {
+    if (FIXED || k <= R) {
       const float wk = w[k];
 #pragma unroll
-      for (int o = 0; o < kStrip; ++o) out[o] = fmaf(wk, x[RMAX + o - k] + x[RMAX + o + k], out[o]);
+      for (int o = 0; o < N; ++o) out[o] = fmaf(wk, x[RMAX + o - k] + x[RMAX + o + k], out[o]);
     }
   }
 }
 
-template <int RMAX>
-__device__ __forceinline__ void strip_load(const float* src, int step, float (&x)[kStrip + 2 * RMAX]) {
-#pragma unroll
-  for (int m = 0; m < kStrip + 2 * RMAX; ++m) x[m] = src[m * step];
+// LDS layout of a column of 256 rows: the rows' even groups of four, then the
+// odd groups.  The y pass reads and writes groups of four rows (16 bytes) with
+// its lanes two groups apart, which in plain order meets every other bank only
+// (measured: 21 conflict cycles per access); here those lanes lie next to each
+// other.  The odd half is turned by 32 words, so that consecutive rows, as the
+// x pass writes and the test reads them, meet different banks too.
+constexpr int kColumn = 256;
+constexpr int kHalf = kColumn / 2;
+__device__ __forceinline__ int even_slot(int pair) { return 4 * pair; }
+__device__ __forceinline__ int odd_slot(int pair) { return kHalf + ((4 * pair + 32) & (kHalf - 1)); }
+__device__ __forceinline__ int row_slot(int r) {
+  return ((r & 4) ? odd_slot(r >> 3) : even_slot(r >> 3)) + (r & 3);
 }
 
-// Tile (blockIdx.x, blockIdx.y) of frame blockIdx.z: interior rows
-// [62 by, 62 by + 62), columns [30 bx, 30 bx + 30); the filtered region adds
-// one pixel around it, the input region R more.
-template <int RMAX>
-__global__ __launch_bounds__(kBlock) void boxer_dog(BoxerArgs a) {
+// Filter and 3 x 3 maxima above minval, one sweep.
+//
+// Block (x, y, z): columns [sweep x, sweep (x + 1)), rows [4 word_rows y, ...)
+// of frame z.  256 threads hold 256 consecutive rows (the contiguous axis),
+// 1 + RMAX of them above the block's first; the block walks right in steps of
+// kStep columns:
+//   x pass: thread t keeps the last 2 RMAX columns of its row in registers,
+//     loads kStep more (256 contiguous bytes per wave and column) and writes
+//     both filtered rows to LDS;
+//   y pass: thread (strip, column) filters 8 rows of one column from LDS in
+//     16-byte reads and writes D to a ring of kRing columns;
+//   test: the columns with both neighbours in the ring, one wave per word,
+//     lanes over rows; a wave goes further only where a pixel exceeds minval.
+// So every input pixel is read once per row band, and D goes to memory only
+// around bright pixels.
+// RS and RL are the two radii, or 0 where they come from `a`.
+//
+// What bounds it: VALU issue (45 of the 70 instructions per pixel are the taps)
+// and the two barriers of a step.  32 frames of 2048 x 2048, boxsize 11: the
+// whole call 0.594 -> 0.303 ms against 0.13 ms for one read of the frames.  The
+// tile kernel before it (62 x 30 pixels, every value of three LDS images read
+// one at a time, D of every pixel written and read back) took 0.54 of 0.60 ms.
+// Suppressing in this kernel, with the halo and the ring that needs, took 0.47:
+// a block then waits for its slowest wave at every candidate.  Filtering the
+// window of each candidate again in boxer_suppress took 0.35, but three times
+// as long as before where a low minval makes one pixel in fifteen a candidate.
+template <int RMAX, int RS, int RL>
+__global__ __launch_bounds__(kBlock) void boxer_detect(BoxerArgs a) {
 #pragma clang fp contract(off)
-  using T = TileLayout<RMAX>;
-  __shared__ float lds[T::kFloats];
-  const int R = a.halo;
+  constexpr int kDRows = kBlock - 2 * RMAX;            // rows of D that are complete
+  // 32 strips, so that half a wave is one column and its 16-byte accesses are
+  // free of conflicts; the last strips' rows past kDRows are filtered from
+  // whatever lies past row 255, and nothing uses them.
+  constexpr int kStrips = kColumn / kStrip;
+  static_assert(kStrips * kStep == kBlock, "y pass layout");
+  static_assert(4 * word_rows_of(RMAX) + 2 <= kDRows && kRing >= kStep + 2, "halo");
+  __shared__ __attribute__((aligned(16))) float lds[(2 * kStep + kRing) * kColumn];
+  float* hs = lds;
+  float* hl = hs + kStep * kColumn;
+  float* ring = hl + kStep * kColumn;
+  constexpr int kWord = word_rows_of(RMAX);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int f = blockIdx.z;
-  const int r0 = blockIdx.y * kWordRows - 1, c0 = blockIdx.x * kInnerCols - 1;   // filtered region origin
-  constexpr int S = T::kStride;
-  float* wgt = lds;
-  float* in = wgt + T::kWeights;                 // [kInCols][S]: column c, row r <-> (c0 + c - RMAX, r0 + r - RMAX)
-  float* hs = in + T::kInCols * S;               // [kDCols][S]: column c, row r <-> (c0 + c, r0 + r - RMAX)
-  float* hl = hs + kDCols * S;
-  float* d = in;                                 // [kDCols][kDStride], reuses `in` after the column pass
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (threadIdx.x <= kMaxRadius) {
-    wgt[threadIdx.x] = a.ws[threadIdx.x];
-    wgt[kMaxRadius + 1 + threadIdx.x] = a.wl[threadIdx.x];
-  }
-  const float* ws = wgt;
-  const float* wl = wgt + kMaxRadius + 1;
+  const int band = blockIdx.y * 4 * kWord;             // first row tested
+  const int first = blockIdx.x * a.sweep;              // first column tested
+  const int last = min(first + a.sweep, a.nx);
   const size_t plane = (size_t)a.ny * a.nx;
-  const float* src = a.frames + (size_t)f * plane;
-  const int lo = RMAX - R, hi_r = RMAX + kDRows + R;
-  // stage the input region (radius RMAX) with replicated edges: every load of
-  // a thread is issued before the first LDS write, so they overlap in flight
-  {
-    constexpr int kIn = T::kInCols * T::kRows;
-    constexpr int kPer = (kIn + kBlock - 1) / kBlock;
-    float v[kPer];
+  const float* src = a.frames + (size_t)f * plane + min(max(band - 1 - RMAX + t, 0), a.ny - 1);
+  const int row0 = band - 1;                           // row of D's index 0
+  const int col0 = first - 1;                          // column of D's ring index 0
+  auto pixel = [&](int c) { return src[(size_t)min(max(c, 0), a.nx - 1) * a.ny]; };
+
+  float x[kStep + 2 * RMAX];
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int e = threadIdx.x + i * kBlock;
-      const int c = e / T::kRows, r = e - c * T::kRows;
-      if (i + 1 < kPer || e < kIn)
-        v[i] = src[(size_t)min(max(c0 + c - RMAX, 0), a.nx - 1) * a.ny + min(max(r0 + r - RMAX, 0), a.ny - 1)];
-    }
+  for (int i = 0; i < kStep + 2 * RMAX; ++i) x[i] = pixel(col0 - RMAX + i);
+  const int steps = (last - first + 2 + kStep - 1) / kStep;
+  const int ys = t % kStrips, yc = t / kStrips;        // y pass: strip and column of the step
+  const int slot = row_slot(t);
+  // the test's row, and the slots of the rows around it in a column of D
+  const int gr = band + wave * kWord + lane;
+  const bool mine = lane < kWord && gr < a.ny;
+  const int own = row_slot(gr - row0), up = row_slot(gr - row0 - 1), down = row_slot(gr - row0 + 1);
+  const bool has_up = gr >= 1, has_down = gr + 1 < a.ny;
+  const float ninf = -__builtin_inff();
+  const int wi = blockIdx.y * 4 + wave;                // word of the column
+  for (int s = 0; s < steps; ++s) {
+    const int base = s * kStep;                        // ring column (not wrapped) of the step's first column
+    {
+      float vs[kStep], vl[kStep];
+      strip_filter<RMAX, RS>(x, a.ws, a.rs, vs);
+      strip_filter<RMAX, RL>(x, a.wl, a.rl, vl);
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int e = threadIdx.x + i * kBlock;
-      const int c = e / T::kRows, r = e - c * T::kRows;
-      if (i + 1 < kPer || e < kIn) in[c * S + r] = v[i];
-    }
-  }
-  __syncthreads();
-  // along x, over rows [lo, hi_r) and 4 strips of 8 columns: first rows
-  // lo..lo+63 (each wave one strip, each lane one row), then the 2R remaining
-  // rows x 4 strips packed onto the fewest lanes (threads 0 .. 8R-1), so the
-  // other waves leave their issue slots to other blocks
-  {
-    auto x_pass = [&](int r, int cb) {
-      float x[T::kStripLen], vs[kStrip], vl[kStrip];
-      strip_load<RMAX>(in + cb * S + r, S, x);
-      strip_filter<RMAX>(x, ws, a.rs, vs);
-      strip_filter<RMAX>(x, wl, a.rl, vl);
-#pragma unroll
-      for (int o = 0; o < kStrip; ++o) {
-        hs[(cb + o) * S + r] = vs[o];
-        hl[(cb + o) * S + r] = vl[o];
+      for (int o = 0; o < kStep; ++o) {
+        hs[o * kColumn + slot] = vs[o];
+        hl[o * kColumn + slot] = vl[o];
       }
-    };
-    x_pass(lo + lane, wave * kStrip);
-    const int t = threadIdx.x;
-    if (t < 4 * (hi_r - lo - 64)) x_pass(lo + 64 + (t >> 2), (t & 3) * kStrip);
-  }
-  __syncthreads();
-  // along y: each thread takes 8 rows of one column (lanes across columns)
-  {
-    const int c = lane & 31, rb = (wave * 2 + (lane >> 5)) * kStrip;
-    float x[T::kStripLen], vs[kStrip], vl[kStrip];
-    strip_load<RMAX>(hs + c * S + rb, 1, x);
-    strip_filter<RMAX>(x, ws, a.rs, vs);
-    strip_load<RMAX>(hl + c * S + rb, 1, x);
-    strip_filter<RMAX>(x, wl, a.rl, vl);
-    // `d` overwrites `in`, which nothing reads after the column pass
+    }
+    // the next step's columns: in flight during the y pass and the test
 #pragma unroll
-    for (int o = 0; o < kStrip; ++o) d[c * T::kDStride + rb + o] = vs[o] - vl[o];
-  }
-  __syncthreads();
-  // one wave per interior column, one lane per region row (rows 1..62 interior)
-  constexpr int DS = T::kDStride;
-  float* dst = a.dog + (size_t)f * plane;
-  for (int cc = 1 + wave; cc <= kInnerCols; cc += kWaves) {
-    const int gc = c0 + cc, gr = r0 + lane;
-    const bool interior = lane >= 1 && lane <= kWordRows && gc < a.nx && gr < a.ny;
-    bool cand = false;
-    if (interior) {
-      const float v = d[cc * DS + lane];
-      dst[(size_t)gc * a.ny + gr] = v;
-      if (v > a.minval) {
-        cand = true;
+    for (int i = 0; i < 2 * RMAX; ++i) x[i] = x[i + kStep];
+    if (s + 1 < steps) {
 #pragma unroll
-        for (int dc = -1; dc <= 1; ++dc) {
-          if (gc + dc < 0 || gc + dc >= a.nx) continue;
+      for (int i = 0; i < kStep; ++i) x[2 * RMAX + i] = pixel(col0 + base + kStep + RMAX + i);
+    }
+    __syncthreads();
+    {
+      float v[kStrip + 2 * RMAX], vs[kStrip], vl[kStrip];
+      auto load = [&](const float* h) {
+        const float* p = h + yc * kColumn;
 #pragma unroll
-          for (int dr = -1; dr <= 1; ++dr) {
-            if (gr + dr < 0 || gr + dr >= a.ny || (dc == 0 && dr == 0)) continue;
-            const float q = d[(cc + dc) * DS + lane + dr];
-            const bool first = dc < 0 || (dc == 0 && dr < 0);
-            if (q > v || (q == v && first)) cand = false;
-          }
+        for (int i = 0; i < (kStrip + 2 * RMAX) / 4; ++i) {   // group 2 ys + i of the column
+          const float4 q = *reinterpret_cast<const float4*>(p + (i & 1 ? odd_slot(ys + i / 2) : even_slot(ys + i / 2)));
+          v[4 * i] = q.x;
+          v[4 * i + 1] = q.y;
+          v[4 * i + 2] = q.z;
+          v[4 * i + 3] = q.w;
         }
+      };
+      load(hs);
+      strip_filter<RMAX, RS>(v, a.ws, a.rs, vs);
+      load(hl);
+      strip_filter<RMAX, RL>(v, a.wl, a.rl, vl);
+      float* d = ring + ((base + yc) & (kRing - 1)) * kColumn;
+      *reinterpret_cast<float4*>(d + even_slot(ys)) =
+          make_float4(vs[0] - vl[0], vs[1] - vl[1], vs[2] - vl[2], vs[3] - vl[3]);
+      *reinterpret_cast<float4*>(d + odd_slot(ys)) =
+          make_float4(vs[4] - vl[4], vs[5] - vl[5], vs[6] - vl[6], vs[7] - vl[7]);
+    }
+    __syncthreads();
+    // Ring columns base - 1 .. base + kStep - 2 have both neighbours.
+    float here[kStep + 2];   // column base - 2 + j (before the first step's: wrapped, not used)
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < kStep + 2; ++j) here[j] = ring[((base - 2 + j) & (kRing - 1)) * kColumn + own];
+#pragma unroll
+    for (int j = 0; j < kStep; ++j) any = any || here[j + 1] > a.minval;
+    uint64_t word = 0;       // lane j: the word of the step's column j
+    if (__ballot(mine && any)) {
+      float above[kStep + 2], below[kStep + 2];
+#pragma unroll
+      for (int j = 0; j < kStep + 2; ++j) {
+        const float* col = ring + ((base - 2 + j) & (kRing - 1)) * kColumn;
+        above[j] = col[up];
+        below[j] = col[down];
+      }
+#pragma unroll
+      for (int j = 0; j < kStep + 2; ++j) {   // out of the frame: -inf, which beats nothing
+        const int gc = col0 + base - 2 + j;
+        const bool in = gc >= 0 && gc < a.nx;
+        above[j] = in && has_up ? above[j] : ninf;
+        below[j] = in && has_down ? below[j] : ninf;
+        here[j] = in ? here[j] : ninf;
+      }
+#pragma unroll
+      for (int j = 0; j < kStep; ++j) {
+        const int gc = col0 + base - 1 + j;
+        const float p = here[j + 1];
+        // the left column and the row above come first in column-major order
+        const float before = fmaxf(fmaxf(fmaxf(above[j], here[j]), below[j]), above[j + 1]);
+        const float after = fmaxf(fmaxf(fmaxf(above[j + 2], here[j + 2]), below[j + 2]), below[j + 1]);
+        const bool cand = mine && gc >= first && gc < last && p > a.minval && !(before >= p) && !(after > p);
+        const uint64_t m = __ballot(cand);
+        word = lane == j ? m | kStored : word;
+        if (mine && gc >= first && gc < last) a.dog[(size_t)f * plane + (size_t)gc * a.ny + gr] = p;
       }
     }
-    const uint64_t word = __ballot(cand) >> 1;
-    if (lane == 0 && gc < a.nx) a.cand[((size_t)f * a.nx + gc) * a.wpc + blockIdx.y] = word;
+    const int gc = col0 + base - 1 + lane;
+    if (lane < kStep && wi < a.wpc && gc >= first && gc < last) a.cand[((size_t)f * a.nx + gc) * a.wpc + wi] = word;
   }
 }
 
@@ -257,63 +299,74 @@ __device__ int64_t block_exclusive_scan(int64_t v, int64_t* sh, int64_t* total) 
   return before + incl - v;
 }
 
-// One word per lane; the wave tests its lanes' candidates one at a time,
-// all 64 lanes reading the candidate's window together.
+// One word per lane; the wave tests its lanes' candidates one at a time, all 64
+// lanes reading the candidate's window together, four elements each at a time
+// so that their reads overlap.
 __global__ __launch_bounds__(kBlock) void boxer_suppress(BoxerArgs a) {
-  __shared__ int64_t sh[kBlock];
+  __shared__ int64_t sh[kWaves];
   const int lane = threadIdx.x & 63;
-  const int64_t w = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const uint64_t m0 = w < a.n_words ? a.cand[w] : 0;
-  uint64_t todo = m0, keep = m0;
-  const int side = 2 * a.win + 1, area = side * side;
-  const int step_c = 64 / side, step_r = 64 - step_c * side;
-  for (;;) {
-    const uint64_t busy = __ballot(todo != 0);
-    if (!busy) break;
-    const int src = __builtin_ctzll(busy);
-    // the candidate: lowest pending bit of lane `src`
-    const uint64_t ms = __shfl(todo, src);
-    const int64_t ws = __shfl(w, src);
-    const int b = __builtin_ctzll(ms);
-    const int wr = (int)(ws % a.wpc);
-    const int64_t fc = ws / a.wpc;
-    const int gc = (int)(fc % a.nx), f = (int)(fc / a.nx);
-    const int gr = wr * kWordRows + b;
-    const float* D = a.dog + (size_t)f * a.ny * a.nx;
-    const float v = D[(size_t)gc * a.ny + gr];
-    bool beaten = false;
-    // window element e = lane + 64 i <-> (column e / side, row e % side), stepped
-    int ec = lane / side, er = lane - ec * side;
-    for (int e = lane; e < area; e += 64) {
-      const int qc = gc - a.win + ec, qr = gr - a.win + er;
-      if (qc >= 0 && qc < a.nx && qr >= 0 && qr < a.ny) {
-        const float q = D[(size_t)qc * a.ny + qr];
-        const bool first = qc < gc || (qc == gc && qr < gr);
-        beaten |= q > v || (q == v && first);
+  const int win = a.win, side = 2 * win + 1, area = side * side;
+  const int inv = (65536 + side - 1) / side;   // e / side = e inv >> 16 for e < 1024, side <= 31
+  const size_t plane = (size_t)a.ny * a.nx;
+  int kept = 0;
+  for (int i = 0; i < a.wpt; ++i) {
+    const int64_t w = ((int64_t)blockIdx.x * a.wpt + i) * kBlock + threadIdx.x;
+    uint64_t todo = w < a.n_words ? a.cand[w] & ~kStored : 0, keep = todo;
+    for (;;) {
+      const uint64_t busy = __ballot(todo != 0);
+      if (!busy) break;
+      const int lead = __builtin_ctzll(busy);
+      // the candidate: lowest pending bit of lane `lead`
+      const uint64_t ms = __shfl(todo, lead);
+      const int64_t ws = __shfl(w, lead);
+      const int b = __builtin_ctzll(ms);
+      const int64_t fc = ws / a.wpc;
+      const int gc = (int)(fc % a.nx), wi = (int)(ws - fc * a.wpc);
+      const int gr = wi * a.word_rows + b;
+      const float* D = a.dog + (size_t)(fc / a.nx) * plane;
+      const float v = D[(size_t)gc * a.ny + gr];
+      // which words of the window's columns are stored: lane l < 32 the upper
+      // word of column gc - win + l, lane 32 + l the lower one (a window is
+      // shorter than a word)
+      const int w_lo = max(gr - win, 0) / a.word_rows, w_hi = min(gr + win, a.ny - 1) / a.word_rows;
+      const int bound = w_hi * a.word_rows;   // first row of the lower word
+      const int sc = (lane & 31) - win;
+      const bool col = (lane & 31) < side && gc + sc >= 0 && gc + sc < a.nx;
+      const uint64_t stored = __ballot(col && (a.cand[(fc + (col ? sc : 0)) * a.wpc + (lane < 32 ? w_lo : w_hi)] >> 63));
+      bool beaten = false;
+      for (int e0 = 0; e0 < area; e0 += 256) {
+        float q[4];
+        bool in[4], before[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int e = e0 + 64 * j + lane, ec = e * inv >> 16, er = e - ec * side;   // column, row of the window
+          const int qc = gc - win + ec, qr = gr - win + er;
+          in[j] = e < area && qr >= 0 && qr < a.ny && ((stored >> (ec + (qr >= bound ? 32 : 0))) & 1);
+          before[j] = ec < win || (ec == win && er < win);
+          q[j] = in[j] ? D[(size_t)qc * a.ny + qr] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) beaten |= in[j] && (q[j] > v || (q[j] == v && before[j]));
+        if (__ballot(beaten)) break;
       }
-      ec += step_c;
-      er += step_r;
-      if (er >= side) {
-        er -= side;
-        ++ec;
+      const bool lost = __ballot(beaten) != 0;
+      if (lane == lead) {
+        todo &= todo - 1;
+        if (lost) keep &= ~(1ull << b);
       }
     }
-    const bool lost = __ballot(beaten) != 0;
-    if (lane == src) {
-      todo &= todo - 1;
-      if (lost) keep &= ~(1ull << b);
-    }
+    if (w < a.n_words) a.keep[w] = keep;
+    kept += __popcll(keep);
   }
-  if (w < a.n_words) a.keep[w] = keep;
   int64_t total;
-  block_exclusive_scan(__popcll(keep), sh, &total);
+  block_exclusive_scan(kept, sh, &total);
   if (threadIdx.x == 0) a.block_base[blockIdx.x] = total;
 }
 
 // Exclusive scan of the per-block counts in place (one block); the total
 // number of detections goes to *count.
 __global__ __launch_bounds__(kScanThreads) void boxer_scan(int64_t* base, int64_t nb, int64_t* count) {
-  __shared__ int64_t sh[kScanThreads];
+  __shared__ int64_t sh[kScanThreads / 64];
   const int t = threadIdx.x;
   const int64_t per = (nb + kScanThreads - 1) / kScanThreads;
   const int64_t lo = min(nb, (int64_t)t * per), hi = min(nb, lo + per);
@@ -329,39 +382,47 @@ __global__ __launch_bounds__(kScanThreads) void boxer_scan(int64_t* base, int64_
   if (t == 0) *count = total;
 }
 
+// The words of one suppress block, wpt consecutive ones per thread, in order;
+// then the block's boxes, one wave each.
 __global__ __launch_bounds__(kBlock) void boxer_place(BoxerArgs a) {
-  __shared__ int64_t sh[kBlock];
-  const int64_t w = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  uint64_t keep = w < a.n_words ? a.keep[w] : 0;
-  int64_t total;
-  int64_t k = a.block_base[blockIdx.x] + block_exclusive_scan(__popcll(keep), sh, &total);
-  if (!keep) return;
-  const int wr = (int)(w % a.wpc);
-  const int64_t fc = w / a.wpc;
-  const int gc = (int)(fc % a.nx), f = (int)(fc / a.nx);
-  const int half = (a.box - 1) / 2;
-  const int c0 = min(max(gc - half, 0), a.nx - a.box);
-  while (keep && k < a.max_boxes) {
-    const int b = __builtin_ctzll(keep);
-    keep &= keep - 1;
-    const int gr = wr * kWordRows + b;
-    const int r0 = min(max(gr - half, 0), a.ny - a.box);
-    a.xc[k] = c0 + 1;
-    a.yc[k] = r0 + 1;
-    a.frame[k] = f + 1;
-    if (a.strength) a.strength[k] = a.dog[((size_t)f * a.nx + gc) * a.ny + gr];
-    ++k;
+  __shared__ int64_t sh[kWaves];
+  const int64_t w0 = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * a.wpt;
+  uint64_t keep[kWordsPerThread];
+  int n = 0;
+#pragma unroll
+  for (int i = 0; i < kWordsPerThread; ++i) {
+    keep[i] = i < a.wpt && w0 + i < a.n_words ? a.keep[w0 + i] : 0;
+    n += __popcll(keep[i]);
   }
-}
-
-__global__ __launch_bounds__(kBlock) void boxer_cut(BoxerArgs a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t n = min(*a.count, a.max_boxes);
-  const int B = a.box, BB = a.box * a.box;
+  int64_t total;
+  const int64_t begin = a.block_base[blockIdx.x];
+  int64_t k = begin + block_exclusive_scan(n, sh, &total);
+  const int B = a.box, BB = a.box * a.box, half = (a.box - 1) / 2;
   const size_t plane = (size_t)a.ny * a.nx;
-  for (int64_t k = (int64_t)blockIdx.x * kWaves + wave; k < n; k += (int64_t)gridDim.x * kWaves) {
-    const float* src = a.frames + (size_t)(a.frame[k] - 1) * plane + (size_t)(a.xc[k] - 1) * a.ny + (a.yc[k] - 1);
-    float* dst = a.rois + (size_t)k * BB;
+  if (n) {
+#pragma unroll
+    for (int i = 0; i < kWordsPerThread; ++i) {
+      const int64_t fc = (w0 + i) / a.wpc;
+      const int wr = (int)((w0 + i) - fc * a.wpc);
+      const int gc = (int)(fc % a.nx), f = (int)(fc / a.nx);
+      const int c0 = min(max(gc - half, 0), a.nx - B);
+      while (keep[i] && k < a.max_boxes) {
+        const int gr = wr * a.word_rows + __builtin_ctzll(keep[i]);
+        keep[i] &= keep[i] - 1;
+        a.xc[k] = c0 + 1;
+        a.yc[k] = min(max(gr - half, 0), a.ny - B) + 1;
+        a.frame[k] = f + 1;
+        if (a.strength) a.strength[k] = a.dog[(size_t)f * plane + (size_t)gc * a.ny + gr];
+        ++k;
+      }
+    }
+  }
+  __syncthreads();   // the corners below are this block's own
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t end = min(begin + total, a.max_boxes);
+  for (int64_t q = begin + wave; q < end; q += kWaves) {
+    const float* src = a.frames + (size_t)(a.frame[q] - 1) * plane + (size_t)(a.xc[q] - 1) * a.ny + (a.yc[q] - 1);
+    float* dst = a.rois + (size_t)q * BB;
     for (int e = lane; e < BB; e += 64) {
       const int col = e / B, row = e - col * B;
       dst[e] = src[(size_t)col * a.ny + row];
@@ -384,22 +445,20 @@ void gaussian_half(double sigma, int R, float* w) {
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// Workspace: D | candidate words | survivor words | block counts.
 struct Layout {
   size_t dog, cand, keep, base, total;
-  int wpc;
-  int64_t n_words, n_blocks;
 };
 
 Layout layout(int ny, int nx, int nf) {
+  // room for the words of either word_rows_of
+  const int64_t n_words = (int64_t)nf * nx * ((ny + word_rows_of(kMaxRadius) - 1) / word_rows_of(kMaxRadius));
   Layout L;
-  L.wpc = (ny + kWordRows - 1) / kWordRows;
-  L.n_words = (int64_t)nf * nx * L.wpc;
-  L.n_blocks = (L.n_words + kBlock - 1) / kBlock;
   L.dog = 0;
   L.cand = L.dog + align256((size_t)ny * nx * nf * sizeof(float));
-  L.keep = L.cand + align256((size_t)L.n_words * sizeof(uint64_t));
-  L.base = L.keep + align256((size_t)L.n_words * sizeof(uint64_t));
-  L.total = L.base + align256((size_t)L.n_blocks * sizeof(int64_t));
+  L.keep = L.cand + align256((size_t)n_words * sizeof(uint64_t));
+  L.base = L.keep + align256((size_t)n_words * sizeof(uint64_t));
+  L.total = L.base + align256((size_t)((n_words + kBlock - 1) / kBlock) * sizeof(int64_t));
   return L;
 }
 
@@ -414,6 +473,15 @@ int check_params(int ny, int nx, int nf, int box, float overlap, float sigma_sma
     return fail(GMLE_ERR_ARG, "sigmas above 4 px are not supported (kernel radius > %d)", kMaxRadius);
   if (isnan(minval)) return fail(GMLE_ERR_ARG, "minval is NaN");
   return GMLE_OK;
+}
+
+// Columns a block sweeps: long sweeps filter little halo (2 columns), short
+// ones give a small stack enough blocks.
+int sweep_columns(const BoxerArgs& a) {
+  const int64_t rows = (int64_t)a.nf * ((a.wpc + 3) / 4);
+  const int64_t parts = std::max<int64_t>(1, kTargetBlocks / rows);   // at most three full rounds
+  const int64_t cols = (a.nx + parts - 1) / parts;
+  return (int)std::min<int64_t>((std::max<int64_t>(cols, kMinSweep) + kStep - 1) / kStep * kStep, 1 << 20);
 }
 
 BoxerArgs make_args(const float* frames, int ny, int nx, int nf, int box, float overlap, float sigma_small,
@@ -431,9 +499,12 @@ BoxerArgs make_args(const float* frames, int ny, int nx, int nf, int box, float 
   a.minval = minval;
   a.win = std::max(1, (int)ceilf((float)box - overlap) - 1);
   a.box = box;
+  a.word_rows = word_rows_of(a.halo);
+  a.wpc = (ny + a.word_rows - 1) / a.word_rows;
+  a.n_words = (int64_t)nf * nx * a.wpc;
+  a.sweep = sweep_columns(a);
+  a.wpt = a.n_words >= kManyWords ? kWordsPerThread : 1;
   const Layout L = layout(ny, nx, nf);
-  a.wpc = L.wpc;
-  a.n_words = L.n_words;
   a.max_boxes = max_boxes;
   char* w = (char*)ws;
   a.dog = (float*)(w + L.dog);
@@ -444,18 +515,24 @@ BoxerArgs make_args(const float* frames, int ny, int nx, int nf, int box, float 
 }
 
 
-int enqueue_boxer(BoxerArgs a, hipStream_t stream) {
-  const Layout L = layout(a.ny, a.nx, a.nf);
-  const dim3 grid((a.nx + kInnerCols - 1) / kInnerCols, L.wpc, a.nf);
-  if (a.halo <= 6)
-    hipLaunchKernelGGL(boxer_dog<6>, grid, dim3(kBlock), 0, stream, a);
+template <int RMAX, int RS, int RL> void launch_detect(const BoxerArgs& a, hipStream_t stream) {
+  const dim3 grid((a.nx + a.sweep - 1) / a.sweep, (a.wpc + 3) / 4, a.nf);
+  hipLaunchKernelGGL((boxer_detect<RMAX, RS, RL>), grid, dim3(kBlock), 0, stream, a);
+}
+
+int enqueue_boxer(const BoxerArgs& a, hipStream_t stream) {
+  // radii 3 and 6 are those of the default sigmas, 1 and 2 px; fixed, the taps
+  // need no branches
+  if (a.rs == 3 && a.rl == 6)
+    launch_detect<6, 3, 6>(a, stream);
+  else if (a.halo <= 6)
+    launch_detect<6, 0, 0>(a, stream);
   else
-    hipLaunchKernelGGL(boxer_dog<kMaxRadius>, grid, dim3(kBlock), 0, stream, a);
-  hipLaunchKernelGGL(boxer_suppress, dim3((unsigned)L.n_blocks), dim3(kBlock), 0, stream, a);
-  hipLaunchKernelGGL(boxer_scan, dim3(1), dim3(kScanThreads), 0, stream, a.block_base, L.n_blocks, a.count);
-  hipLaunchKernelGGL(boxer_place, dim3((unsigned)L.n_blocks), dim3(kBlock), 0, stream, a);
-  const int64_t cut = std::min<int64_t>(kCutBlocks, std::max<int64_t>(1, (a.max_boxes + kWaves - 1) / kWaves));
-  if (a.max_boxes > 0) hipLaunchKernelGGL(boxer_cut, dim3((unsigned)cut), dim3(kBlock), 0, stream, a);
+    launch_detect<kMaxRadius, 0, 0>(a, stream);
+  const int64_t n_blocks = (a.n_words + (int64_t)kBlock * a.wpt - 1) / ((int64_t)kBlock * a.wpt);
+  hipLaunchKernelGGL(boxer_suppress, dim3((unsigned)n_blocks), dim3(kBlock), 0, stream, a);
+  hipLaunchKernelGGL(boxer_scan, dim3(1), dim3(kScanThreads), 0, stream, a.block_base, n_blocks, a.count);
+  if (a.max_boxes > 0) hipLaunchKernelGGL(boxer_place, dim3((unsigned)n_blocks), dim3(kBlock), 0, stream, a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? GMLE_OK : hip_fail(e, "kernel launch");
 }

@@ -247,6 +247,29 @@ def test_find_boxes_matches_oracle_bit_for_bit(name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ny,nx,nf,box,overlap,sigmas,minval", [
+    (16, 16, 3, 16, 0.0, (1.0, 2.0), -np.inf),     # smaller than one word, window wider than the frame
+    (61, 25, 2, 7, 2.0, (1.0, 2.0), 0.0),          # one row into the second word; one column into a second sweep
+    (241, 130, 2, 11, 2.0, (1.0, 2.0), 1.0),       # one row into the second band
+    (299, 49, 1, 3, 0.5, (0.34, 0.5), -np.inf),    # radii 1 and 2, windows of 5 and less
+    (113, 90, 2, 9, 2.0, (3.9, 1.0), -2.0),        # radius 12 (56-row words), small and large exchanged
+    (225, 31, 2, 16, 0.0, (4.0, 4.1), -np.inf),    # radius 12 twice, a row into the second band of 56-row words
+    (16, 2048, 256, 16, 8.0, (1.0, 2.0), 4.0),     # many words: four per thread
+])
+def test_find_boxes_at_the_edges_of_the_sweep(ny, nx, nf, box, overlap, sigmas, minval):
+    """Noise with ties (whole-number pixels), where windows cross words, bands,
+    sweeps and frame edges: counts, places, strengths and pixels equal the
+    oracle's."""
+    rng = np.random.default_rng(ny * nx)
+    frames = np.asfortranarray(rng.poisson(20.0, (ny, nx, nf)).astype(np.float32))
+    want = refboxer.find(frames, box, overlap, sigmas[0], sigmas[1], minval)
+    got = gbx.find_boxes(frames, box, overlap, sigmas[0], sigmas[1], minval)
+    print(f"[boxer] {ny}x{nx}x{nf}: {want['n']} detections", flush=True)
+    _assert_same(got, want, "edges")
+    assert got["n"] > 0
+
+
+@pytest.mark.gpu
 def test_find_boxes_truncates_at_capacity():
     frames, _ = spots_stack(128, 128, 2, 25, seed=20)
     want = refboxer.find(frames, 7, 2.0, 1.0, 2.0, 4.0)
