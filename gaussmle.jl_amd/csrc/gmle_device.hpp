@@ -46,7 +46,11 @@ __device__ __forceinline__ float dpp_swap2(float v) { return dpp_move<kDppSwap2>
 __device__ __forceinline__ double dpp_swap1(double v) { return dpp_move<kDppSwap1>(v); }
 __device__ __forceinline__ double dpp_swap2(double v) { return dpp_move<kDppSwap2>(v); }
 
+// No contraction here: a product that the caller passes in would otherwise be
+// fused into the first add, fma(a, b, neighbour's rounded a b), which differs
+// between the two lanes.
 template <int L, class T> __device__ __forceinline__ T group_sum(T v) {
+#pragma clang fp contract(off)
   static_assert(L == 1 || L == 2 || L == 4 || L == 8 || L == 16, "lanes per ROI must be 1, 2, 4, 8 or 16");
   if constexpr (L >= 2) v = v + dpp_move<kDppSwap1>(v);
   if constexpr (L >= 4) v = v + dpp_move<kDppSwap2>(v);

@@ -34,6 +34,7 @@
 namespace gmle {
 
 constexpr float kErfK = 1.2011224031448364f;   // sqrt(log2 e): v = k u
+constexpr float kErfRate = 0.84932180028801904f;   // k / sqrt 2 (k / (sigma sqrt 2) scales an edge's distance)
 constexpr float kErfC = 3.0028059482574463f;   // c = k * 2.5: t = 0 at |u| = 2.5
 constexpr float kErfC2 = 6.005611896514893f;   // 2 c (exact)
 

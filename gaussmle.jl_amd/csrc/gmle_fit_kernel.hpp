@@ -16,12 +16,12 @@
 //     stay in VGPRs for every Newton iteration and the final pass.
 //   * The model is separable: value = bg + N*Phix[j]*Phiy[i].  Per iteration
 //     each axis needs only N+1 edge evaluations (one erf and one exp each)
-//     instead of the reference's 4 erf + 4-8 exp per pixel; every per-pixel
-//     gradient / diagonal-Hessian term is a product of a column table and a row
-//     table, so the per-pixel work is one reciprocal plus about ten FMAs that
-//     feed per-column accumulators.  Column totals are folded into the P
-//     gradient and P diagonal-Hessian sums, which are summed across the L lanes
-//     with DPP permutes.
+//     instead of the reference's 4 erf + 4-8 exp per pixel, and every gradient,
+//     diagonal-Hessian and Fisher term is a product of a column value, a row
+//     value and a pixel weight.  A pixel therefore only feeds a few weighted
+//     column and row sums (accumulate); the tables multiply those sums.  Row
+//     values are shared through LDS (publish_rows).  The P gradient and P
+//     diagonal-Hessian values are summed across the L lanes with DPP permutes.
 //   * The Newton update (exact division, step clamp, box clamp) is replicated
 //     on the L lanes so they stay bit-identical.
 //   * PREC_FP32 computes the final pass (LLR, full Fisher matrix, inversion,
@@ -81,6 +81,15 @@ template <> struct DM<float> {
   // (1 ulp) and a multiply instead of the ~10-instruction IEEE division.
   // The Newton step keeps the IEEE division.
   static __device__ __forceinline__ float div(float a, float b) { return a * fast_rcp(b); }
+  // 1 / b: v_rcp_f32 and one Newton step (correctly rounded but for rare last
+  // bits), left out where the reciprocal is not finite.
+  static __device__ __forceinline__ float inv(float b) {
+    const float r = fast_rcp(b);
+    const float e = fmaf(-b, r, 1.f);
+    return fabsf(e) < 1.f ? fmaf(e, r, r) : r;
+  }
+  // The scale t -> v of an edge, k / (sigma sqrt 2).
+  static __device__ __forceinline__ float erf_rate(float, float inv_s) { return inv_s * kErfRate; }
 };
 template <> struct DM<double> {
   static __device__ __forceinline__ double erf_scale() { return 1.0; }
@@ -95,6 +104,8 @@ template <> struct DM<double> {
   }
   static __device__ __forceinline__ double inv_sqrt_2pi() { return kInvSqrt2PiD; }
   static __device__ __forceinline__ double div(double a, double b) { return a / b; }
+  static __device__ __forceinline__ double inv(double b) { return 1.0 / b; }
+  static __device__ __forceinline__ double erf_rate(double sigma, double) { return sqrt(0.5 / (sigma * sigma)); }
 };
 
 // ---------------------------------------------------------------------------
@@ -153,8 +164,15 @@ __device__ __forceinline__ void axis_tables(T mu, T sigma, T nph, int first, Axi
 
 // Axis constants of axis_tables() and single-edge evaluation, for computing
 // one pixel's tables from its two edges on the fly (column side).
+// The constants past c and 1/sigma are formed where they are used: an
+// iteration needs them only after its pixel loop, where four values held
+// across the loop would take registers from it.
 template <class T> struct AxisK {
-  T mu, s_erf, c, c2, cs, css, m2s;
+  T mu, s_erf, c, inv_s;
+  __device__ __forceinline__ T c2() const { return c * inv_s * inv_s; }
+  __device__ __forceinline__ T cs() const { return c * inv_s; }
+  __device__ __forceinline__ T css() const { return c2() * inv_s * inv_s; }
+  __device__ __forceinline__ T m2s() const { return T(-2) * inv_s; }
 };
 template <class T> struct Edge {
   T se, hs, g, tg, t3g;   // signed erfc, half-sign (gmle_erf.hpp), Gaussian, t g, t^3 g
@@ -162,14 +180,10 @@ template <class T> struct Edge {
 template <class T>
 __device__ __forceinline__ AxisK<T> axis_consts(T mu, T sigma, T nph) {
   AxisK<T> k;
-  const T inv_s = DM<T>::div(T(1), sigma);
+  k.inv_s = DM<T>::inv(sigma);
   k.mu = mu;
-  k.s_erf = sqrt(DM<T>::div(T(0.5), sigma * sigma)) * DM<T>::erf_scale();
-  k.c = -nph * DM<T>::inv_sqrt_2pi() * inv_s;
-  k.c2 = k.c * inv_s * inv_s;
-  k.cs = k.c * inv_s;
-  k.css = k.c2 * inv_s * inv_s;
-  k.m2s = T(-2) * inv_s;
+  k.s_erf = DM<T>::erf_rate(sigma, k.inv_s);
+  k.c = -nph * DM<T>::inv_sqrt_2pi() * k.inv_s;
   return k;
 }
 template <class T, bool SIG>
@@ -191,122 +205,205 @@ __device__ __forceinline__ Pix<T> pix_from_edges(const AxisK<T>& k, const Edge<T
   p.phi = pixel_integral<T>(lo.se, lo.hs, hi.se, hi.hs);
   p.D = k.c * (hi.g - lo.g);
   const T w = hi.tg - lo.tg;
-  p.D2 = k.c2 * w;
-  p.S = SIG ? k.cs * w : T(0);
-  p.SS = SIG ? k.m2s * p.S + k.css * (hi.t3g - lo.t3g) : T(0);
+  p.D2 = k.c2() * w;
+  p.S = SIG ? k.cs() * w : T(0);
+  p.SS = SIG ? k.m2s() * p.S + k.css() * (hi.t3g - lo.t3g) : T(0);
   return p;
 }
 
 // ---------------------------------------------------------------------------
-// Row tables shared by the L lanes of an ROI.  Every lane needs every row's
-// tables, but evaluating the N + 1 row edges (one erf and one exp each) on
-// all L lanes repeats the same work L times.  Instead lane r evaluates edges
-// r, r + L, r + 2L, ... (slot s holds edge r + L s) and builds the tables of
-// rows r, r + L, ...; a row's tables reach the other lanes by a DPP
-// broadcast from its owner where they are used.  Row r + L s's upper edge is
-// lane r + 1's slot-s edge, or lane 0's slot-(s + 1) edge for the group's
-// last lane: lane 0 offers its next edge, the others their current one, and
-// every lane reads the next lane's offer.  Each value comes from the same
-// expressions as in the replicated evaluation; the compiler's FMA contraction
-// can still round a rare one differently, so a kernel and its replicated twin
-// may differ in the last bit of an ROI's result.
+// One pixel row or column of an axis as plain differences of its two edges.
+// The tables of axis_tables() are these times the axis constants:
+//   D = c dg,  D2 = c2 w,  S = cs w,  SS = m2s cs w + css t3
+// so sums weighted with them need the constants once per iteration, not once
+// per row.
 // ---------------------------------------------------------------------------
-// Where sharing is used (gfx950 register counts): sharing keeps a few more
-// values live, so the tiles at the top of each two-wave range keep the
-// replicated evaluation: with 4 lanes the largest box that fits 256 VGPRs
-// (max_box_within_256), with 2 lanes the two largest, since the multi-shape
-// kernel, which calls every 1-, 2- and 4-lane tile, has to stay at two waves
-// per SIMD too.  From 8 lanes up every tile shares.
-template <int MODEL, int CAM, int N, int L> constexpr bool share_rows() {
-  if (L == 1) return false;
-  if (L >= 8) return true;
-  if (L == 2) return N + 1 < max_box_within_256(MODEL, CAM, L);
-  return N != max_box_within_256(MODEL, CAM, L);
+template <class T> struct Band {
+  T phi, dg, w, t3;
+};
+template <class T, bool SIG>
+__device__ __forceinline__ Edge<T> edge_at(const AxisK<T>& k, T pos) {
+  Edge<T> r;
+  const T t = pos - k.mu;
+  DM<T>::erf_gauss(t, k.s_erf, r.se, r.hs, r.g);
+  r.tg = t * r.g;
+  r.t3g = SIG ? t * t * r.tg : T(0);
+  return r;
+}
+template <class T, bool SIG>
+__device__ __forceinline__ Band<T> band_from_edges(const Edge<T>& lo, const Edge<T>& hi) {
+  Band<T> b;
+  b.phi = pixel_integral<T>(lo.se, lo.hs, hi.se, hi.hs);
+  b.dg = hi.g - lo.g;
+  b.w = hi.tg - lo.tg;
+  b.t3 = SIG ? hi.t3g - lo.t3g : T(0);
+  return b;
 }
 
+// What the pixel loop and the row folds read of one row.
+struct RowVals {
+  float phi, phi2, pw, dg, w, t3, dg2, w2;   // phi^2, phi w, dg^2, w^2
+};
+template <bool SIG> __device__ __forceinline__ RowVals row_vals(const Band<float>& b) {
+  RowVals v;
+  v.phi = b.phi;
+  v.phi2 = b.phi * b.phi;
+  v.dg = b.dg;
+  v.w = b.w;
+  v.dg2 = b.dg * b.dg;
+  v.pw = SIG ? b.phi * b.w : 0.f;
+  v.t3 = SIG ? b.t3 : 0.f;
+  v.w2 = SIG ? b.w * b.w : 0.f;
+  return v;
+}
+
+// ---------------------------------------------------------------------------
+// Row tables shared by the L lanes of an ROI.  Every lane needs every row's
+// values, but evaluating the N + 1 row edges (one erf and one exp each) on all
+// L lanes repeats the same work L times.  Instead lane r evaluates the rows
+// [r RS, r RS + RS) and writes them to LDS, from where every lane of the ROI
+// reads a row's values (one or two 16-byte reads at one address per ROI) when
+// its loop reaches the row.  LDS reads issue beside the VALU, where the DPP
+// moves used before took 5 VALU instructions per row at 2 and 4 lanes and 15
+// at 8.  The wave is its own only reader, and LDS operations of a wave stay in
+// order, so no barrier is needed beyond the compiler's.  An ROI's rows take
+// RS L slots (slots past row N - 1 are written and never read) plus 4 words,
+// which spread the ROIs that one 16-lane phase of a read serves over the banks.
+// ---------------------------------------------------------------------------
 template <int N, int L> constexpr int row_slots() { return (N + L - 1) / L; }   // rows per lane
-template <int N, int L> constexpr int edge_slots() { return (N + L) / L; }     // edges 0..N per lane
+// Words of a row: its eight values with a width, four without.  One lane per
+// ROI keeps four of the eight and forms the products again.
+template <int MODEL, int L> constexpr int row_words() { return (MT<MODEL>::EXTRA != 0 && L > 1) ? 8 : 4; }
+// Words from one row to the next: one lane per ROI interleaves the wave's 64
+// ROIs, so that a read takes consecutive addresses.
+template <int MODEL, int L> constexpr int row_stride() { return L == 1 ? 4 * kWave : row_words<MODEL, L>(); }
+template <int MODEL, int N, int L> constexpr int roi_words() {
+  return row_slots<N, L>() * L * row_words<MODEL, L>() + 4;
+}
+template <int MODEL, int N, int L> constexpr int rows_words() {
+  return L == 1 ? N * 4 * kWave : kWave / L * roi_words<MODEL, N, L>();
+}
+// WORDS words of LDS; every caller with the same WORDS in a kernel gets the
+// same array.
+template <int WORDS> __device__ __forceinline__ float* wave_lds() {
+  __shared__ float4 words[WORDS / 4];
+  return reinterpret_cast<float*>(words);
+}
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// This lane's rows, evaluated and written to its ROI's LDS words.
+template <int MODEL, int N, int L>
+__device__ __forceinline__ void publish_rows(const AxisK<float>& ky, int r, float* roi) {
+  constexpr bool SIG = MT<MODEL>::EXTRA != 0;
+  constexpr int RS = row_slots<N, L>();
+  constexpr int W = row_stride<MODEL, L>();
+  const float r0 = (float)(r * RS);
+  float* dst = roi + r * RS * W;
+  wave_lds_order();   // after the previous evaluation's reads
+  Edge<float> lo = edge_at<float, SIG>(ky, r0 + 0.5f);
+#pragma unroll
+  for (int s = 0; s < RS; ++s) {
+    const Edge<float> hi = edge_at<float, SIG>(ky, r0 + ((float)s + 1.5f));
+    const RowVals v = row_vals<SIG>(band_from_edges<float, SIG>(lo, hi));
+    lo = hi;
+    float4* q = reinterpret_cast<float4*>(dst + s * W);
+    if constexpr (SIG && L > 1) {
+      q[0] = make_float4(v.phi, v.phi2, v.pw, v.dg);
+      q[1] = make_float4(v.w, v.t3, v.dg2, v.w2);
+    } else {
+      q[0] = make_float4(v.phi, v.dg, v.w, SIG ? v.t3 : v.dg2);
+    }
+  }
+  wave_lds_order();
+}
+
+// Row i of the ROI, from LDS.
+template <int MODEL, int L> __device__ __forceinline__ RowVals read_row(const float* roi, int i) {
+  constexpr bool SIG = MT<MODEL>::EXTRA != 0;
+  const float4* src = reinterpret_cast<const float4*>(roi + i * row_stride<MODEL, L>());
+  const float4 a = src[0];
+  if constexpr (SIG && L > 1) {
+    const float4 b = src[1];
+    return RowVals{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  } else if constexpr (SIG) {
+    return row_vals<true>(Band<float>{a.x, a.y, a.z, a.w});
+  } else {
+    return RowVals{a.x, a.x * a.x, 0.f, a.y, a.z, 0.f, a.w, 0.f};
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Tail split.  With N = L q + 1 the plain column blocks give each lane
 // ceil(N / L) = q + 1 columns, and the group computes L (q + 1) columns for N:
 // almost a whole padding column per lane (13 px on 4 lanes: 52 pixel slots
 // per lane for 169 pixels).  Split instead, each lane holds q full columns
-// [r q, r q + q) and, of the last column N - 1, the rows r, r + L, r + 2L, ...
-// -- exactly the rows whose tables the lane builds itself when rows are
-// shared, so those pixels need no broadcast: q N + ceil(N / L) slots (13 px on
-// 4 lanes: 43).  The last column's partial row sums are folded with that
-// column's tables on every lane and summed across the group with the rest
-// (the fold is linear in the sums).
+// [r q, r q + q) and, of the last column N - 1, the rows it evaluates itself: q N + ceil(N / L) slots (13 px on 4 lanes:
+// 43).  The last column's partial sums are folded with that column's values on
+// every lane and summed across the group with the rest (the fold is linear).
 // ---------------------------------------------------------------------------
-template <int MODEL, int CAM, int N, int L> constexpr bool tail_split() {
-  return L >= 2 && N > L && N % L == 1 && N <= kMaxSmallBox && share_rows<MODEL, CAM, N, L>();
-}
+// From 4 lanes up: with 2 lanes a padding column is one in N + 1 and costs less
+// than the tail's own row folds (XYNBS 11 px on 2 lanes, with the split 1.55 ns
+// per ROI, as much as 12 px).
+template <int N, int L> constexpr bool tail_split() { return L >= 4 && N > L && N % L == 1; }
 // Register-resident full columns per lane.
-template <int MODEL, int CAM, int N, int L> constexpr int block_cols() {
-  return tail_split<MODEL, CAM, N, L>() ? N / L : (N + L - 1) / L;
+template <int N, int L> constexpr int block_cols() {
+  return tail_split<N, L>() ? N / L : (N + L - 1) / L;
 }
-
-template <int L, bool SIG>
-__device__ __forceinline__ Pix<float> slot_row(const AxisK<float>& kr, int r, const Edge<float>& e_s,
-                                               const Edge<float>& e_next) {
-  const bool first = r == 0;
-  Edge<float> hi;
-  hi.se = group_next<L>(first ? e_next.se : e_s.se);
-  hi.hs = group_next<L>(first ? e_next.hs : e_s.hs);
-  hi.g = group_next<L>(first ? e_next.g : e_s.g);
-  hi.tg = group_next<L>(first ? e_next.tg : e_s.tg);
-  hi.t3g = SIG ? group_next<L>(first ? e_next.t3g : e_s.t3g) : 0.f;
-  return pix_from_edges<float, SIG>(kr, e_s, hi);
+// Rows whose pixel work the scheduler may mix: a row of few columns is a short
+// dependent chain (model, reciprocal, weights, sums), so several go together.
+// About four pixels: sCMOS XYNBS 13 px (3 columns) runs 2.30 ms per 1M ROIs one
+// row at a time and 2.36 two rows together; 100 ROIs of 7 px (one column) run
+// 25.0 us one row at a time and 24.3 together.
+template <int CB> constexpr int rows_together() { return CB >= 4 ? 1 : 4 / CB; }
+// Least waves per SIMD a fit kernel is built for: three where a lane's pixels (and
+// variances) leave the loop enough of the 168 VGPRs that three waves have, and
+// three waves' LDS fits a CU's 160 KB, else two where a few spilled values
+// reach them (sCMOS XYNBS 16 px on 4 lanes, 128 values, needs 258 VGPRs: 4.19
+// against 2.93 ms per 1M ROIs at one wave and two).  Above the first line the
+// spills cost more than the third wave hides: sCMOS XYNBS 13 px
+// on 4 lanes (86 values) runs 2.46 -> 2.34 ms per 1M ROIs with three waves and
+// 164 B of scratch, XYNB 11 px on one lane (121 values) 1.51 -> 2.04 ms.
+constexpr int kLds3Waves = 160 * 1024 / 12, kLds2Waves = 160 * 1024 / 8;
+template <int MODEL, int CAM, int N, int L> constexpr int min_waves() {
+  constexpr int px = (block_cols<N, L>() * N + (tail_split<N, L>() ? row_slots<N, L>() : 0)) * (CAM == SCMOS ? 2 : 1);
+  return px <= 88 && rows_words<MODEL, N, L>() * 4 <= kLds3Waves ? 3 : px <= 144 ? 2 : 1;
 }
-
-// The edge of slot s + 1 when some lane has one (else unused).
-template <int N, int L, bool SIG>
-__device__ __forceinline__ Edge<float> next_slot_edge(const AxisK<float>& kr, int r, int s, const Edge<float>& e_s) {
-  return (s + 1 < edge_slots<N, L>()) ? edge_eval<float, SIG>(kr, r + L * (s + 1)) : e_s;
+// The pixel loop reads only phi (and phi^2) of a column; its other values wait
+// in LDS until the fold, one quad per column and lane, where there is room for
+// them beside the rows.
+template <int MODEL, int CAM, int N, int L> constexpr int park_words() {
+  constexpr int w = block_cols<N, L>() * (MT<MODEL>::EXTRA != 0 ? 4 : 2) * kWave;
+  constexpr int room = min_waves<MODEL, CAM, N, L>() == 3 ? kLds3Waves : kLds2Waves;
+  return (rows_words<MODEL, N, L>() + w) * 4 <= room ? w : 0;
 }
-
-// Row i's tables on every lane of the group, from lane o = i mod L.  o is a
-// constant once the caller's row loop is unrolled, so the chain of tests
-// folds to a single broadcast.
-template <int L, bool SIG, int O = 0>
-__device__ __forceinline__ Pix<float> bcast_pix(const Pix<float>& p, int o) {
-  if constexpr (O + 1 < L) {
-    if (o != O) return bcast_pix<L, SIG, O + 1>(p, o);
+// LDS words of one wave.
+template <int MODEL, int CAM, int N, int L> constexpr int wave_words() {
+  return rows_words<MODEL, N, L>() + park_words<MODEL, CAM, N, L>();
+}
+template <bool SIG> __device__ __forceinline__ void park_band(float* park, int cc, const Band<float>& b) {
+  if constexpr (SIG) {
+    reinterpret_cast<float4*>(park)[cc * kWave] = make_float4(b.dg, b.w, b.t3, 0.f);
+  } else {
+    reinterpret_cast<float2*>(park)[cc * kWave] = make_float2(b.dg, b.w);
   }
-  Pix<float> q;
-  q.phi = group_bcast<L, O>(p.phi);
-  q.D = group_bcast<L, O>(p.D);
-  q.D2 = group_bcast<L, O>(p.D2);
-  q.S = SIG ? group_bcast<L, O>(p.S) : 0.f;
-  q.SS = SIG ? group_bcast<L, O>(p.SS) : 0.f;
-  return q;
+}
+template <bool SIG> __device__ __forceinline__ Band<float> parked_band(const float* park, int cc, float phi) {
+  if constexpr (SIG) {
+    const float4 q = reinterpret_cast<const float4*>(park)[cc * kWave];
+    return Band<float>{phi, q.x, q.y, q.z};
+  } else {
+    const float2 q = reinterpret_cast<const float2*>(park)[cc * kWave];
+    return Band<float>{phi, q.x, q.y, 0.f};
+  }
 }
 
-// All N rows' tables on every lane, as axis_tables() builds them; own[s]
-// receives this lane's own row r + L s (the tail split uses them).
-template <int N, int L, bool SIG>
-__device__ __forceinline__ void shared_axis_tables(const AxisK<float>& kr, int r, AxisTab<float, N>& tb,
-                                                   Pix<float>* own) {
-  constexpr int RS = row_slots<N, L>();
-  Edge<float> e_s = edge_eval<float, SIG>(kr, r);
-#pragma unroll
-  for (int s = 0; s < RS; ++s) {
-    const Edge<float> e_next = next_slot_edge<N, L, SIG>(kr, r, s, e_s);
-    own[s] = slot_row<L, SIG>(kr, r, e_s, e_next);
-    e_s = e_next;
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const Pix<float> q = bcast_pix<L, SIG>(own[i / L], i % L);
-    tb.phi[i] = q.phi;
-    tb.D[i] = q.D;
-    tb.D2[i] = q.D2;
-    if constexpr (SIG) {
-      tb.S[i] = q.S;
-      tb.SS[i] = q.SS;
-    }
-  }
+// Whether block column cc lies past the ROI on some lane (L does not divide
+// N).  Such a column carries zero column values and adds nothing.
+template <int N, int L> constexpr bool may_pad(int cc) {
+  return !tail_split<N, L>() && (L - 1) * block_cols<N, L>() + cc >= N;
 }
 
 // Per-ROI width parameters for one evaluation of the model.
@@ -355,78 +452,23 @@ __device__ __forceinline__ void model_widths(const T* th, const float* psf, Widt
   }
 }
 
-// Fold one column's row-weighted sums S[0..10] = S1..S11 (see accumulate)
-// into the gradient / diagonal Hessian with the column's tables
-// (unified_kernel.jl:330-333): grad_k += dudt_k cf, H_k += d2_k cf - dudt_k^2 df.
-template <int MODEL>
-__device__ __forceinline__ void fold_column(const Pix<float>& cx, const Widths<float>& w, const float* S, float* G,
-                                            float* H) {
-  using Tr = MT<MODEL>;
-  constexpr bool SIG = Tr::EXTRA != 0;
-  constexpr bool TWO = (Tr::EXTRA == 1 || Tr::EXTRA == 3);
-  const float px = cx.phi, Dx = cx.D, D2x = cx.D2;
-  G[Tr::IX] += Dx * S[0];
-  H[Tr::IX] += D2x * S[0] - Dx * Dx * S[1];
-  G[Tr::IY] += px * S[2];
-  H[Tr::IY] += px * S[3] - px * px * S[4];
-  G[Tr::IN] += px * S[0];
-  H[Tr::IN] -= px * px * S[1];
-  G[Tr::IBG] += S[5];
-  H[Tr::IBG] -= S[6];
-  if constexpr (SIG) {
-    float ax, aax;
-    if constexpr (MODEL == ASTIG) {
-      ax = w.dsx * cx.S;
-      aax = cx.SS * (w.dsx * w.dsx) + cx.S * w.d2sx;
-    } else {
-      ax = cx.S;
-      aax = cx.SS;
-    }
-    if constexpr (TWO) {
-      G[Tr::IE1] += ax * S[0] + px * S[7];
-      H[Tr::IE1] += aax * S[0] + px * S[8] - ax * ax * S[1] - 2.f * ax * px * S[9] - px * px * S[10];
-    } else {
-      G[Tr::IE1] += ax * S[0];
-      H[Tr::IE1] += aax * S[0] - ax * ax * S[1];
-      G[Tr::IE2] += px * S[7];
-      H[Tr::IE2] += px * S[8] - px * px * S[10];
-    }
-  }
-}
-
-// One pixel of the tail column (tail split): row ry of this lane's slot,
-// column tables folded later.  ok is false for slots past the last row; their
-// terms are zero.  For the Poisson fast path rs[] collects the row sums the q
-// form subtracts (phi, D, D2, A, AA, rows).
-template <int MODEL, int CAM, bool FAST>
-__device__ __forceinline__ void tail_pixel(const Pix<float>& ry, const Widths<float>& w, float d, float var, bool ok,
-                                           float ncx, float bg, float* St, float* rs) {
-  using Tr = MT<MODEL>;
-  constexpr bool SIG = Tr::EXTRA != 0;
-  constexpr bool TWO = (Tr::EXTRA == 1 || Tr::EXTRA == 3);
-  float ay = 0.f, aay = 0.f;
-  if constexpr (SIG) {
-    if constexpr (MODEL == ASTIG) {
-      ay = w.dsy * ry.S;
-      aay = ry.SS * (w.dsy * w.dsy) + ry.S * w.d2sy;
-    } else {
-      ay = ry.S;
-      aay = ry.SS;
-    }
-  }
-  const float py = ry.phi;
-  const float mu = fmaf(ncx, py, bg);
-  float cf, df;
+// One pixel's likelihood weights (camera_models.jl:19-42): cf multiplies the
+// model's derivatives in the gradient, df in the Hessian.  FAST (Poisson
+// only): every model value exceeds 0.01 and neither 1e4 cap can bind; then
+// cf = d/mu - 1 and df = d/mu^2 = (cf + 1)/mu are one FMA each.
+template <int CAM, bool FAST>
+__device__ __forceinline__ void pixel_weights(float d, float var, float mu, float& cf, float& df) {
   if constexpr (CAM == IDEAL) {
     const float rc = fast_rcp(mu);
-    const float q = d * rc;
     if constexpr (FAST) {
-      cf = q;
-      df = q * rc;
+      cf = fmaf(d, rc, -1.f);
+      df = fmaf(cf, rc, rc);
     } else {
+      const float q = d * rc;
       const bool pos = mu > 0.01f;   // camera_models.jl:23-32
-      cf = pos ? jmin(q - 1.f, 1.0e4f) : 0.f;
-      df = pos ? jmin(q * rc, 1.0e4f) : 0.f;
+      const float a = q - 1.f, b = q * rc;
+      cf = pos ? (1.0e4f < a ? 1.0e4f : a) : 0.f;   // Julia's min: a NaN passes
+      df = pos ? (1.0e4f < b ? 1.0e4f : b) : 0.f;
     }
   } else {
     const float v = mu + var;   // camera_models.jl:36-42
@@ -434,312 +476,214 @@ __device__ __forceinline__ void tail_pixel(const Pix<float>& ry, const Widths<fl
     cf = (d - mu) * rc;
     df = rc;
   }
-  cf = ok ? cf : 0.f;
-  df = ok ? df : 0.f;
-  St[0] = fmaf(py, cf, St[0]);
-  St[1] = fmaf(py * py, df, St[1]);
-  St[2] = fmaf(ry.D, cf, St[2]);
-  St[3] = fmaf(ry.D2, cf, St[3]);
-  St[4] = fmaf(ry.D * ry.D, df, St[4]);
-  St[5] += cf;
-  St[6] += df;
-  if constexpr (SIG) {
-    St[7] = fmaf(ay, cf, St[7]);
-    St[8] = fmaf(aay, cf, St[8]);
-    St[10] = fmaf(ay * ay, df, St[10]);
-    if constexpr (TWO) St[9] = fmaf(py * ay, df, St[9]);
-  }
-  if constexpr (CAM == IDEAL && FAST) {
-    rs[0] += ok ? py : 0.f;
-    rs[1] += ok ? ry.D : 0.f;
-    rs[2] += ok ? ry.D2 : 0.f;
-    rs[3] += ok ? ay : 0.f;
-    rs[4] += ok ? aay : 0.f;
-    rs[5] += ok ? 1.f : 0.f;
-  }
 }
 
-// The tail column's sums folded into G / H with its tables tl.
-template <int MODEL, int CAM, bool FAST>
-__device__ __forceinline__ void tail_fold(float* St, const float* rs, const Pix<float>& tl, const Widths<float>& w,
-                                          float* G, float* H) {
-  if constexpr (CAM == IDEAL && FAST) {
-    St[0] -= rs[0];
-    St[2] -= rs[1];
-    St[3] -= rs[2];
-    St[5] -= rs[5];
-    if constexpr (MT<MODEL>::EXTRA != 0) {
-      St[7] -= rs[3];
-      St[8] -= rs[4];
-    }
-  }
-  fold_column<MODEL>(tl, w, St, G, H);
-}
-
-// The same sums with rows in the outer loop: each row's tables are built on
-// the fly from its two edges and the CB columns of this lane keep their S
-// vectors live instead.  Cheaper in VGPRs than holding every row's tables
-// when there are many row tables (sigma / z models) and few columns per lane.
-template <int MODEL, int CAM, int N, int L, bool FAST, bool SHARE>
-__device__ __forceinline__ void accumulate_rows(const float* dv, const float* vr, const float* dt, const float* vt,
-                                                int c0, float nph, float bg, const AxisK<float>& kr, int r,
-                                                const AxisK<float>& kc, const Widths<float>& w, float* G, float* H) {
-  using Tr = MT<MODEL>;
-  constexpr int P = Tr::P;
-  constexpr bool TAIL = tail_split<MODEL, CAM, N, L>();
-  constexpr int CB = block_cols<MODEL, CAM, N, L>();
-  constexpr bool SIG = Tr::EXTRA != 0;
-  constexpr bool TWO = (Tr::EXTRA == 1 || Tr::EXTRA == 3);
-  constexpr int NS = SIG ? 11 : 7;
-  static_assert(!TAIL || SHARE, "the tail split uses the lane's own row tables");
-#pragma unroll
-  for (int k = 0; k < P; ++k) { G[k] = 0.f; H[k] = 0.f; }
-  // this lane's column tables (and the tail column's, from lane L - 1, whose
-  // block ends at edge N - 1)
-  Pix<float> cx[CB];
-  float ncx[CB];
-  Pix<float> tl{};
-  {
-    Edge<float> lo = edge_eval<float, SIG>(kc, c0);
-#pragma unroll
-    for (int cc = 0; cc < CB; ++cc) {
-      const Edge<float> hi = edge_eval<float, SIG>(kc, c0 + cc + 1);
-      cx[cc] = pix_from_edges<float, SIG>(kc, lo, hi);
-      lo = hi;
-      ncx[cc] = nph * cx[cc].phi;
-    }
-    if constexpr (TAIL) {
-      const Edge<float> hi = edge_eval<float, SIG>(kc, N);
-      tl = bcast_pix<L, SIG>(pix_from_edges<float, SIG>(kc, lo, hi), L - 1);
-    }
-  }
-  const float ncx_t = nph * tl.phi;
-  float St[11], rs[6];
-#pragma unroll
-  for (int q = 0; q < 11; ++q) St[q] = 0.f;
-#pragma unroll
-  for (int q = 0; q < 6; ++q) rs[q] = 0.f;
-  float S[CB][11];
-#pragma unroll
-  for (int cc = 0; cc < CB; ++cc)
-#pragma unroll
-    for (int q = 0; q < 11; ++q) S[cc][q] = 0.f;
-  float sphi = 0.f, sD = 0.f, sD2 = 0.f, sA = 0.f, sAA = 0.f;
-  // Without sharing, rlo is the running lower edge.  With it, rlo is this
-  // lane's edge of the current slot, and `own` the tables of its row in that
-  // slot, built when the group reaches the slot's first row.
-  Edge<float> rlo = edge_eval<float, SIG>(kr, SHARE ? r : 0);
-  Pix<float> own;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    // Keep each row's work together: without this the scheduler hoists later
-    // rows' edge evaluations and every row's tables become live at once.
-    __builtin_amdgcn_sched_barrier(0);
-    Pix<float> ry;
-    if constexpr (!SHARE) {
-      const Edge<float> rhi = edge_eval<float, SIG>(kr, i + 1);
-      ry = pix_from_edges<float, SIG>(kr, rlo, rhi);
-      rlo = rhi;
-    } else {
-      if (i % L == 0) {
-        const Edge<float> e_next = next_slot_edge<N, L, SIG>(kr, r, i / L, rlo);
-        own = slot_row<L, SIG>(kr, r, rlo, e_next);
-        rlo = e_next;
-        // the tail pixel of this slot's row r + i, with the lane's own tables
-        if constexpr (TAIL)
-          tail_pixel<MODEL, CAM, FAST>(own, w, dt[i / L], CAM == SCMOS ? vt[i / L] : 0.f, r + i < N, ncx_t, bg, St,
-                                       rs);
-      }
-      ry = bcast_pix<L, SIG>(own, i % L);
-    }
-    float ay = 0.f, aay = 0.f;
-    if constexpr (SIG) {
-      if constexpr (MODEL == ASTIG) {
-        ay = w.dsy * ry.S;
-        aay = ry.SS * (w.dsy * w.dsy) + ry.S * w.d2sy;
-      } else {
-        ay = ry.S;
-        aay = ry.SS;
-      }
-    }
-    if constexpr (CAM == IDEAL && FAST) {
-      sphi += ry.phi;
-      sD += ry.D;
-      sD2 += ry.D2;
-      if constexpr (SIG) { sA += ay; sAA += aay; }
-    }
-    const float py = ry.phi, py2 = py * py, Dy2 = ry.D * ry.D, a2 = ay * ay, pa = py * ay;
-#pragma unroll
-    for (int cc = 0; cc < CB; ++cc) {
-      const float d = dv[cc * N + i];
-      const float mu = fmaf(ncx[cc], py, bg);
-      float cf, df;
-      if constexpr (CAM == IDEAL) {
-        const float rc = fast_rcp(mu);
-        const float q = d * rc;
-        if constexpr (FAST) {
-          cf = q;   // cf + 1; the constant is removed after the row sums
-          df = q * rc;
-        } else {
-          const bool ok = mu > 0.01f;   // camera_models.jl:23-32
-          cf = ok ? jmin(q - 1.f, 1.0e4f) : 0.f;
-          df = ok ? jmin(q * rc, 1.0e4f) : 0.f;
-        }
-      } else {
-        const float v = mu + vr[cc * N + i];   // camera_models.jl:36-42
-        const float rc = fast_rcp(v);
-        cf = (d - mu) * rc;
-        df = rc;
-      }
-      S[cc][0] = fmaf(py, cf, S[cc][0]);
-      S[cc][1] = fmaf(py2, df, S[cc][1]);
-      S[cc][2] = fmaf(ry.D, cf, S[cc][2]);
-      S[cc][3] = fmaf(ry.D2, cf, S[cc][3]);
-      S[cc][4] = fmaf(Dy2, df, S[cc][4]);
-      S[cc][5] += cf;
-      S[cc][6] += df;
-      if constexpr (SIG) {
-        S[cc][7] = fmaf(ay, cf, S[cc][7]);
-        S[cc][8] = fmaf(aay, cf, S[cc][8]);
-        S[cc][10] = fmaf(a2, df, S[cc][10]);
-        if constexpr (TWO) S[cc][9] = fmaf(pa, df, S[cc][9]);
-      }
-    }
-    // With shared rows, also tie this row's sums to the end of the row, or
-    // the pixel work of every row sinks below the last row's broadcast.
-    if constexpr (SHARE) {
-#pragma unroll
-      for (int cc = 0; cc < CB; ++cc) {
-        asm volatile("" : "+v"(S[cc][0]), "+v"(S[cc][1]), "+v"(S[cc][2]), "+v"(S[cc][3]), "+v"(S[cc][4]),
-                     "+v"(S[cc][5]), "+v"(S[cc][6]));
-        if constexpr (SIG) asm volatile("" : "+v"(S[cc][7]), "+v"(S[cc][8]), "+v"(S[cc][10]));
-        if constexpr (TWO) asm volatile("" : "+v"(S[cc][9]));
-      }
-    }
-  }
+// This lane's column values, and with the tail split those of the last column
+// (from lane L - 1, whose block ends at edge N - 1).
+template <int N, int L, bool SIG>
+__device__ __forceinline__ void column_bands(const AxisK<float>& kx, int c0, Band<float>* cb, Band<float>& tl) {
+  constexpr int CB = block_cols<N, L>();
+  const float f0 = (float)c0;
+  Edge<float> lo = edge_at<float, SIG>(kx, f0 + 0.5f);
 #pragma unroll
   for (int cc = 0; cc < CB; ++cc) {
-    if constexpr (CAM == IDEAL && FAST) {
-      S[cc][0] -= sphi;
-      S[cc][2] -= sD;
-      S[cc][3] -= sD2;
-      S[cc][5] -= (float)N;
-      if constexpr (SIG) { S[cc][7] -= sA; S[cc][8] -= sAA; }
-    }
-    // Columns past the ROI (last lane of a group when L does not divide N)
-    // contribute nothing.  Selects, not a branch: a per-lane branch here
-    // splits the block and costs ~100 VGPRs of live ranges.
-    const bool cvalid = (L == 1) || TAIL || (c0 + cc < N);
-#pragma unroll
-    for (int q = 0; q < 11; ++q) S[cc][q] = cvalid ? S[cc][q] : 0.f;
-    fold_column<MODEL>(cx[cc], w, S[cc], G, H);
+    const Edge<float> hi = edge_at<float, SIG>(kx, f0 + ((float)cc + 1.5f));
+    cb[cc] = band_from_edges<float, SIG>(lo, hi);
+    lo = hi;
+    if (may_pad<N, L>(cc) && c0 + cc >= N) cb[cc] = Band<float>{0.f, 0.f, 0.f, 0.f};
   }
-  if constexpr (TAIL) tail_fold<MODEL, CAM, FAST>(St, rs, tl, w, G, H);
-  (void)NS;
-}
-
-// Loop order with the smaller live-register estimate: column-outer holds every
-// row's tables (5 per row, 9 with sigma / z terms, 8 for separate sigmas);
-// row-outer holds this lane's column tables and S vectors (about 11 and 18
-// per column).
-template <int MODEL, int CAM, int N, int L> constexpr bool row_outer() {
-  constexpr int CB = (N + L - 1) / L;
-  constexpr int ex = MT<MODEL>::EXTRA;
-  constexpr int row_tables = ex == 0 ? 5 : (ex == 2 ? 8 : 9);
-  constexpr int per_col = ex == 0 ? 11 : 18;
-  return per_col * CB < row_tables * N;
+  if constexpr (tail_split<N, L>()) {
+    const Band<float> b = band_from_edges<float, SIG>(lo, edge_at<float, SIG>(kx, (float)N + 0.5f));
+    tl.phi = group_bcast<L, L - 1>(b.phi);
+    tl.dg = group_bcast<L, L - 1>(b.dg);
+    tl.w = group_bcast<L, L - 1>(b.w);
+    tl.t3 = SIG ? group_bcast<L, L - 1>(b.t3) : 0.f;
+  }
 }
 
 // ---------------------------------------------------------------------------
 // One Newton iteration's gradient G[P] and diagonal Hessian H[P] over this
-// lane's column block (unified_kernel.jl:319-334):
+// lane's pixels (unified_kernel.jl:319-334):
 //   G_k = sum_ij dudt_k cf,   H_k = sum_ij (d2udt2_k cf - dudt_k^2 df).
-// Each per-pixel term factors as (column table)(row table)(cf or df), so the
-// pixel loop only accumulates row-weighted cf / df sums per column
-//   S1 = sum_i phiy cf    S2 = sum_i phiy^2 df   S3 = sum_i Dy cf
-//   S4 = sum_i D2y cf     S5 = sum_i Dy^2 df     S6 = sum_i cf    S7 = sum_i df
-//   S8 = sum_i Ay cf      S9 = sum_i AAy cf      S10 = sum_i phiy Ay df
-//   S11 = sum_i Ay^2 df
-// (A = derivative w.r.t. the sigma / z parameter on the row axis, AA its second
-// derivative) that are then multiplied by the column's tables, which are built
-// from the column's two edges on the fly.
-// FAST (Poisson only): every model value exceeds 0.01 and neither 1e4 cap
-// (camera_models.jl:23-28) can bind, so cf + 1 = data/model is accumulated and
-// the constant row sums (sphi, sD, ...) are subtracted once per column.
+// Every term factors as (column value)(row value)(cf or df), so the pixels
+// only feed six sums (seven where one parameter moves both widths):
+//   C_j = sum_i phiy_i cf     CC_j = sum_i phiy_i^2 df      per column
+//   R_i = sum_j phix_j cf     RR_i = sum_j phix_j^2 df      per row
+//   sum cf, sum df            X_j = sum_i phiy_i wy_i df    per column
+// and the derivatives of the x axis weight C and CC, those of the y axis R and
+// RR: d/dx is sum_j Dx_j C_j, d/dy is sum_i Dy_i R_i, and so on.  Weighting
+// the pixels with every row table instead took 7 (fixed width) to 11 sums per
+// pixel and held them all per column.  Rows run in the outer loop: a row's R
+// and RR are folded as soon as the row ends, and a lane keeps only its
+// columns' five values and three sums.
+// Bound by VALU issue.  gfx950, ms per launch against 7 to 11 sums per pixel
+// with the row tables by DPP: sCMOS XYNBS 13 px, 1M ROIs 3.20 -> 2.36; astigmatic
+// 15 px, 1M 6.07 -> 3.96; XYNBS 21 px, 200K 1.80 -> 1.02; XYNB 11 px on one lane,
+// 1M 1.386 -> 1.369.
 // ---------------------------------------------------------------------------
 template <int MODEL, int CAM, int N, int L, bool FAST>
-__device__ __forceinline__ void accumulate(const float* dv, const float* vr, int c0, float nph, float bg,
-                                           const AxisTab<float, N>& ry, const AxisK<float>& kc,
-                                           const Widths<float>& w, const float* Ay, const float* AAy,
-                                           float sphi, float sD, float sD2, float sA, float sAA, float* G,
+__device__ __forceinline__ void accumulate(const float* dv, const float* vr, const float* dt, const float* vt, int c0,
+                                           int r, float nph, float bg, const AxisK<float>& kx, const AxisK<float>& ky,
+                                           const Widths<float>& w, const float* roi, float* park, float* G,
                                            float* H) {
   using Tr = MT<MODEL>;
-  constexpr int P = Tr::P;
-  constexpr bool TAIL = tail_split<MODEL, CAM, N, L>();
-  constexpr int CB = block_cols<MODEL, CAM, N, L>();
+  constexpr bool TAIL = tail_split<N, L>();
+  constexpr int CB = block_cols<N, L>();
+  constexpr int RS = row_slots<N, L>();
   constexpr bool SIG = Tr::EXTRA != 0;
   constexpr bool TWO = (Tr::EXTRA == 1 || Tr::EXTRA == 3);
+  constexpr int KR = rows_together<CB>();
+  Band<float> cb[CB], tl{};
+  column_bands<N, L, SIG>(kx, c0, cb, tl);
+  constexpr bool PARK = park_words<MODEL, CAM, N, L>() != 0;
+  if constexpr (PARK) {
 #pragma unroll
-  for (int k = 0; k < P; ++k) { G[k] = 0.f; H[k] = 0.f; }
-  Edge<float> lo = edge_eval<float, SIG>(kc, c0);
+    for (int cc = 0; cc < CB; ++cc) park_band<SIG>(park, cc, cb[cc]);
+    wave_lds_order();
+  }
+  float px2[CB], C[CB], CC[CB], X[TWO ? CB : 1], pad_cf[CB], pad_df[CB];
 #pragma unroll
   for (int cc = 0; cc < CB; ++cc) {
-    const Edge<float> hi = edge_eval<float, SIG>(kc, c0 + cc + 1);
-    const Pix<float> cx = pix_from_edges<float, SIG>(kc, lo, hi);
-    lo = hi;
-    const bool cvalid = (L == 1) || TAIL || (c0 + cc < N);
-    const float nphx = nph * cx.phi;
-    float S1 = 0.f, S2 = 0.f, S3 = 0.f, S4 = 0.f, S5 = 0.f, S6 = 0.f, S7 = 0.f;
-    float S8 = 0.f, S9 = 0.f, S10 = 0.f, S11 = 0.f;
+    px2[cc] = cb[cc].phi * cb[cc].phi;
+    C[cc] = CC[cc] = 0.f;
+    pad_cf[cc] = pad_df[cc] = 0.f;
+    if constexpr (TWO) X[cc] = 0.f;
+  }
+  float y1 = 0.f, y2 = 0.f, y3 = 0.f, y4 = 0.f, y5 = 0.f;   // dg R, w R, t3 R, dg^2 RR, w^2 RR over the rows
+  float scf = 0.f, sdf = 0.f;
+  auto fold_row = [&](const RowVals& v, float R, float RR) __attribute__((always_inline)) {
+    y1 = fmaf(v.dg, R, y1);
+    y2 = fmaf(v.w, R, y2);
+    y4 = fmaf(v.dg2, RR, y4);
+    if constexpr (SIG) {
+      y3 = fmaf(v.t3, R, y3);
+      y5 = fmaf(v.w2, RR, y5);
+    }
+  };
+  float a1 = 0.f, a2 = 0.f, a3 = 0.f, a4 = 0.f, a5 = 0.f, gn = 0.f, hn = 0.f, xs = 0.f;
+  auto fold_col = [&](const Band<float>& b, float b2, float c, float cc2, float x) __attribute__((always_inline)) {
+    a1 = fmaf(b.dg, c, a1);
+    a2 = fmaf(b.w, c, a2);
+    a3 = fmaf(b.dg * b.dg, cc2, a3);
+    gn = fmaf(b.phi, c, gn);
+    hn = fmaf(b2, cc2, hn);
+    if constexpr (SIG) {
+      a4 = fmaf(b.t3, c, a4);
+      a5 = fmaf(b.w * b.w, cc2, a5);
+      if constexpr (TWO) xs = fmaf(b.phi * b.w, x, xs);
+    }
+  };
+  if constexpr (TAIL) {
+    // the last column's pixels of this lane's own rows (slots past the last
+    // row weigh nothing)
+    const float npx = nph * tl.phi, tp2 = tl.phi * tl.phi;
+    float Ct = 0.f, CCt = 0.f, Xt = 0.f;
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const float d = dv[cc * N + i];
-      const float mu = fmaf(nphx, ry.phi[i], bg);
+    for (int s = 0; s < RS; ++s) {
+      if (s % KR == 0) __builtin_amdgcn_sched_barrier(0);
+      const RowVals v = read_row<MODEL, L>(roi, r * RS + s);
+      const float mu = fmaf(npx, v.phi, bg);
       float cf, df;
-      if constexpr (CAM == IDEAL) {
-        const float rc = fast_rcp(mu);
-        const float q = d * rc;
-        if constexpr (FAST) {
-          cf = q;   // cf + 1; the constant is removed after the row sums
-          df = q * rc;
-        } else {
-          const bool ok = mu > 0.01f;   // camera_models.jl:23-32
-          cf = ok ? jmin(q - 1.f, 1.0e4f) : 0.f;
-          df = ok ? jmin(q * rc, 1.0e4f) : 0.f;
-        }
+      pixel_weights<CAM, FAST>(dt[s], CAM == SCMOS ? vt[s] : 0.f, mu, cf, df);
+      if ((L - 1) * RS + s >= N) {   // some lane's slot lies past the last row
+        const bool ok = r * RS + s < N;
+        cf = ok ? cf : 0.f;
+        df = ok ? df : 0.f;
+      }
+      Ct = fmaf(v.phi, cf, Ct);
+      CCt = fmaf(v.phi2, df, CCt);
+      if constexpr (TWO) Xt = fmaf(v.pw, df, Xt);
+      fold_row(v, tl.phi * cf, tp2 * df);
+      scf += cf;
+      sdf += df;
+    }
+    fold_col(tl, tp2, Ct, CCt, Xt);
+    // done here, not where the sums are next used
+    asm volatile("" : "+v"(a1), "+v"(a2), "+v"(a3), "+v"(gn), "+v"(hn), "+v"(y1), "+v"(y2), "+v"(y4), "+v"(scf),
+                 "+v"(sdf));
+    if constexpr (SIG) asm volatile("" : "+v"(a4), "+v"(a5), "+v"(y3), "+v"(y5), "+v"(xs));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // Row i's values are read from LDS during row i - 1.
+  RowVals next = read_row<MODEL, L>(roi, 0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    // Keep the rows' work apart: without this the scheduler hoists later rows'
+    // values and pixel products and they all become live at once.
+    if (i % KR == 0) __builtin_amdgcn_sched_barrier(0);
+    const RowVals v = next;
+    if (i + 1 < N) next = read_row<MODEL, L>(roi, i + 1);
+    const float pn = nph * v.phi;
+    float R = 0.f, RR = 0.f;
+#pragma unroll
+    for (int cc = 0; cc < CB; ++cc) {
+      const float mu = fmaf(cb[cc].phi, pn, bg);
+      float cf, df;
+      pixel_weights<CAM, FAST>(dv[cc * N + i], CAM == SCMOS ? vr[cc * N + i] : 0.f, mu, cf, df);
+      C[cc] = fmaf(v.phi, cf, C[cc]);
+      CC[cc] = fmaf(v.phi2, df, CC[cc]);
+      if constexpr (TWO) X[cc] = fmaf(v.pw, df, X[cc]);
+      R = cc == 0 ? cb[cc].phi * cf : fmaf(cb[cc].phi, cf, R);
+      RR = cc == 0 ? px2[cc] * df : fmaf(px2[cc], df, RR);
+      // A padding pixel has data 0; its weights are 0 under sCMOS (infinite
+      // variance), and are dropped after the rows for the ideal camera.
+      if (CAM == IDEAL && may_pad<N, L>(cc)) {
+        pad_cf[cc] += cf;
+        pad_df[cc] += df;
       } else {
-        const float v = mu + vr[cc * N + i];   // camera_models.jl:36-42
-        const float rc = fast_rcp(v);
-        cf = (d - mu) * rc;
-        df = rc;
-      }
-      const float py = ry.phi[i];
-      S1 = fmaf(py, cf, S1);
-      S2 = fmaf(py * py, df, S2);
-      S3 = fmaf(ry.D[i], cf, S3);
-      S4 = fmaf(ry.D2[i], cf, S4);
-      S5 = fmaf(ry.D[i] * ry.D[i], df, S5);
-      S6 += cf;
-      S7 += df;
-      if constexpr (SIG) {
-        S8 = fmaf(Ay[i], cf, S8);
-        S9 = fmaf(AAy[i], cf, S9);
-        S11 = fmaf(Ay[i] * Ay[i], df, S11);
-        if constexpr (TWO) S10 = fmaf(py * Ay[i], df, S10);
+        scf += cf;
+        sdf += df;
       }
     }
-    if constexpr (CAM == IDEAL && FAST) {
-      S1 -= sphi;
-      S3 -= sD;
-      S4 -= sD2;
-      S6 -= (float)N;
-      if constexpr (SIG) { S8 -= sA; S9 -= sAA; }
+    fold_row(v, R, RR);
+    // ... and tie this row's sums to the end of the row, or instruction
+    // selection sinks the pixel work of every row below the last one.
+    if (i % KR != KR - 1) continue;
+#pragma unroll
+    for (int cc = 0; cc < CB; ++cc) {
+      asm volatile("" : "+v"(C[cc]), "+v"(CC[cc]));
+      if constexpr (TWO) asm volatile("" : "+v"(X[cc]));
+      if (CAM == IDEAL && may_pad<N, L>(cc)) asm volatile("" : "+v"(pad_cf[cc]), "+v"(pad_df[cc]));
     }
-    // Columns past the ROI contribute nothing (selects, not a branch).
-    const float Sv[11] = {cvalid ? S1 : 0.f, cvalid ? S2 : 0.f, cvalid ? S3 : 0.f, cvalid ? S4 : 0.f,
-                          cvalid ? S5 : 0.f, cvalid ? S6 : 0.f, cvalid ? S7 : 0.f, cvalid ? S8 : 0.f,
-                          cvalid ? S9 : 0.f, cvalid ? S10 : 0.f, cvalid ? S11 : 0.f};
-    fold_column<MODEL>(cx, w, Sv, G, H);
+    asm volatile("" : "+v"(y1), "+v"(y2), "+v"(y4), "+v"(scf), "+v"(sdf));
+    if constexpr (SIG) asm volatile("" : "+v"(y3), "+v"(y5));
+  }
+#pragma unroll
+  for (int cc = 0; cc < CB; ++cc) {
+    fold_col(PARK ? parked_band<SIG>(park, cc, cb[cc].phi) : cb[cc], px2[cc], C[cc], CC[cc],
+             TWO ? X[TWO ? cc : 0] : 0.f);
+    if (CAM == IDEAL && may_pad<N, L>(cc)) {
+      scf += c0 + cc < N ? pad_cf[cc] : 0.f;
+      sdf += c0 + cc < N ? pad_df[cc] : 0.f;
+    }
+  }
+  G[Tr::IX] = kx.c * a1;
+  H[Tr::IX] = kx.c2() * a2 - (kx.c * kx.c) * a3;
+  G[Tr::IY] = ky.c * y1;
+  H[Tr::IY] = ky.c2() * y2 - (ky.c * ky.c) * y4;
+  G[Tr::IN] = gn;
+  H[Tr::IN] = -hn;
+  G[Tr::IBG] = scf;
+  H[Tr::IBG] = -sdf;
+  if constexpr (SIG) {
+    // width terms of each axis: first derivative ex w, second (m2s + d2) w + css t3
+    const float csx = kx.cs() * a2, csy = ky.cs() * y2;                       // sum S C, sum S R
+    const float ssx = kx.m2s() * csx + kx.css() * a4, ssy = ky.m2s() * csy + ky.css() * y3;   // sum SS C, sum SS R
+    const float qx = kx.cs() * kx.cs() * a5, qy = ky.cs() * ky.cs() * y5;         // sum S^2 CC, sum S^2 RR
+    const float qxy = 2.f * (kx.cs() * ky.cs()) * xs;
+    if constexpr (MODEL == XYNBS) {
+      G[Tr::IE1] = csx + csy;
+      H[Tr::IE1] = ssx + ssy - qx - qy - qxy;
+    } else if constexpr (MODEL == XYNBSXSY) {
+      G[Tr::IE1] = csx;
+      H[Tr::IE1] = ssx - qx;
+      G[Tr::IE2] = csy;
+      H[Tr::IE2] = ssy - qy;
+    } else {
+      G[Tr::IE1] = w.dsx * csx + w.dsy * csy;
+      H[Tr::IE1] = (w.dsx * w.dsx) * (ssx - qx) + w.d2sx * csx + (w.dsy * w.dsy) * (ssy - qy) + w.d2sy * csy -
+                   (w.dsx * w.dsy) * qxy;
+    }
   }
 }
 
@@ -754,8 +698,6 @@ template <int N, bool SC> struct RegSrc {
   static constexpr bool kInRegisters = true;
   const float* dv;   // this lane's column block, [cc * N + i]
   const float* vr;
-  const float* dt = nullptr;   // tail split: this lane's rows r + L s of the last column
-  const float* vt = nullptr;
   __device__ __forceinline__ float d(int cc, int i) const { return dv[cc * N + i]; }
   __device__ __forceinline__ float var(int cc, int i) const { return SC ? vr[cc * N + i] : 0.f; }
   __device__ __forceinline__ void column(int cc, float* dcol, float* vcol) const {
@@ -901,12 +843,12 @@ __device__ __forceinline__ FinalOut<TF, P> final_reduce(TF* Fu, TF llr) {
   return out;
 }
 
-template <int MODEL, int CAM, int N, int L, class TF, class Src, bool TAIL = false>
+template <int MODEL, int CAM, int N, int L, class TF, class Src>
 __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass(const float* th, const float* psf, int c0,
-                                                               const Src& src, int r = 0) {
+                                                               const Src& src) {
   using Tr = MT<MODEL>;
   constexpr int P = Tr::P;
-  constexpr int CB = TAIL ? N / L : (N + L - 1) / L;
+  constexpr int CB = (N + L - 1) / L;
   constexpr bool SIG = Tr::EXTRA != 0;
   TF thf[P];
 #pragma unroll
@@ -929,7 +871,7 @@ __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass(const float* th
     const Pix<TF> fx = pix_from_edges<TF, SIG>(kf, flo, fhi);
     flo = fhi;
     const TF px = fx.phi;
-    const bool cvalid = (L == 1) || TAIL || (c0 + cc < N);
+    const bool cvalid = (L == 1) || (c0 + cc < N);
     TF ax = TF(0);
     if constexpr (SIG) ax = (MODEL == ASTIG) ? wf.dsx * fx.S : fx.S;
     float dcol[N], vcol[CAM == SCMOS ? N : 1];
@@ -954,25 +896,6 @@ __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass(const float* th
     // in flight.
 #pragma unroll 1
     for (int cc = 0; cc < CB; ++cc) column(cc);
-  }
-  if constexpr (TAIL) {
-    // this lane's rows r + L s of the last column, tables from their edges
-    static_assert(Src::kInRegisters, "tail pixels are register-resident");
-    const Pix<TF> fx = pix_from_edges<TF, SIG>(kf, edge_eval<TF, false>(kf, N - 1), edge_eval<TF, false>(kf, N));
-    const AxisK<TF> ky = axis_consts<TF>(thf[Tr::IY], wf.sy, nphf);
-    TF ax = TF(0);
-    if constexpr (SIG) ax = (MODEL == ASTIG) ? wf.dsx * fx.S : fx.S;
-#pragma unroll
-    for (int s = 0; s < row_slots<N, L>(); ++s) {
-      const int ri = r + L * s;
-      const Pix<TF> ry = pix_from_edges<TF, SIG>(ky, edge_eval<TF, false>(ky, ri), edge_eval<TF, false>(ky, ri + 1));
-      TF ay = TF(0);
-      if constexpr (SIG) ay = (MODEL == ASTIG) ? wf.dsy * ry.S : ry.S;
-      TF du[P];
-      final_du<MODEL, TF>(fx.phi, ry.phi, fx.D, ry.D, ax, ay, du);
-      const TF mu = bgf + nphf * fx.phi * ry.phi;
-      final_pixel<CAM, P, TF>((TF)src.dt[s], CAM == SCMOS ? (TF)src.vt[s] : TF(0), mu, du, ri < N, Fu, llr);
-    }
   }
   return final_reduce<L, P, TF>(Fu, llr);
 }
@@ -1035,6 +958,318 @@ __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass_rows(const floa
   return final_reduce<L, P, TF>(Fu, llr);
 }
 
+// One pixel's LLR term lp (camera_models.jl:60-85) and Fisher weight wv: 1/v
+// where the model is > 0, else 0 (v = model, or model + variance for sCMOS).
+template <int CAM, class T> __device__ __forceinline__ void final_weights(T d, T var, T mu, T& lp, T& wv) {
+  constexpr bool F32 = sizeof(T) == 4;
+  if constexpr (CAM == IDEAL) {
+    // camera_models.jl:60-71, as d log(mu/d) + d - mu with one log:
+    // d log(mu/d) = -d log(d (1/mu)), and 1/mu is also the Fisher weight.
+    // Float32 takes 1/mu from v_rcp_f32 (1 ulp); the single log also avoids
+    // the cancellation of d log(mu) against d log(d) in the two-log form.
+    if constexpr (F32) {
+      // ln x as v_log_f32 (log2) times ln 2.  x = d/mu of a pixel with d > 0
+      // lies far above the denormal range; the clamp keeps even a denormal
+      // product finite (its term is then ~0, as it would be).
+      wv = mu > T(0) ? fast_rcp(mu) : T(0);
+      const float x = fmaxf(d * wv, 1.17549435e-38f);
+      const float lnx = __builtin_amdgcn_logf(x) * 0.693147180559945309f;
+      lp = (mu > T(0) && d >= T(0)) ? -d * lnx + (d - mu) : T(0);   // -mu at d = 0 (lnx is finite there)
+    } else {
+      wv = mu > T(0) ? T(1) / mu : T(0);
+      lp = (mu > T(0) && d > T(0)) ? -d * log(d * wv) + (d - mu) : (mu > T(0) && d == T(0)) ? -mu : T(0);
+    }
+  } else {
+    const T v = mu + var;   // camera_models.jl:73-85
+    const T res = d - mu;
+    const T rv = T(1) / v;
+    lp = v > T(0) ? T(-0.5) * (res * res * rv) : T(0);
+    wv = mu > T(0) ? rv : T(0);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The Fisher matrix sum_ij du_k du_l wv (unified_kernel.jl:378-396) from
+// weighted sums, as accumulate() forms the gradient: with the column sums
+//   C = sum_i phiy wv, CC = sum_i phiy^2 wv, Y = sum_i phiy dgy wv, Z = sum_i phiy wy wv
+// and the row sums R, RR, every entry is a sum over columns or rows.  Six sums
+// per pixel (seven with a width) take the place of the P derivatives and the
+// P (P + 1) / 2 products.
+// ---------------------------------------------------------------------------
+template <class T> struct FisherSums {
+  T x = 0, xx = 0, xn = 0, n = 0, nn = 0, xy = 0;                        // columns
+  T w = 0, xw = 0, nw = 0, ww = 0, xz = 0, wy = 0, wz = 0;               // columns, width terms
+  T ry = 0, ryy = 0, ryn = 0, rw = 0, ryw = 0, rnw = 0, rww = 0;         // rows
+  T s = 0;                                                               // sum of the weights
+  template <bool SIG> __device__ __forceinline__ void column(const Band<T>& b, T C, T CC, T Y, T Z) {
+    const T gp = b.dg * b.phi;
+    x += b.dg * C;
+    xx += b.dg * b.dg * CC;
+    xn += gp * CC;
+    n += b.phi * C;
+    nn += b.phi * b.phi * CC;
+    xy += gp * Y;
+    if constexpr (SIG) {
+      const T pw = b.phi * b.w;
+      w += b.w * C;
+      xw += b.dg * b.w * CC;
+      nw += pw * CC;
+      ww += b.w * b.w * CC;
+      xz += gp * Z;
+      wy += pw * Y;
+      wz += pw * Z;
+    }
+  }
+  template <bool SIG> __device__ __forceinline__ void row(const Band<T>& b, T R, T RR) {
+    ry += b.dg * R;
+    ryy += b.dg * b.dg * RR;
+    ryn += b.dg * b.phi * RR;
+    if constexpr (SIG) {
+      rw += b.w * R;
+      ryw += b.dg * b.w * RR;
+      rnw += b.phi * b.w * RR;
+      rww += b.w * b.w * RR;
+    }
+  }
+};
+// The upper triangle Fu (k <= l, row by row) from the sums and the axis
+// constants: D = c dg, and the width or z derivative of an axis is e w.
+template <int MODEL, class T>
+__device__ __forceinline__ void fisher_entries(const FisherSums<T>& f, const AxisK<T>& kx, const AxisK<T>& ky,
+                                               const Widths<T>& wd, T* Fu) {
+  using Tr = MT<MODEL>;
+  constexpr int P = Tr::P;
+  auto set = [&](int k, int l, T v) __attribute__((always_inline)) {
+    const int a = k < l ? k : l, b = k < l ? l : k;
+    Fu[a * P - a * (a - 1) / 2 + (b - a)] = v;
+  };
+  set(Tr::IX, Tr::IX, kx.c * kx.c * f.xx);
+  set(Tr::IX, Tr::IY, kx.c * ky.c * f.xy);
+  set(Tr::IX, Tr::IN, kx.c * f.xn);
+  set(Tr::IX, Tr::IBG, kx.c * f.x);
+  set(Tr::IY, Tr::IY, ky.c * ky.c * f.ryy);
+  set(Tr::IY, Tr::IN, ky.c * f.ryn);
+  set(Tr::IY, Tr::IBG, ky.c * f.ry);
+  set(Tr::IN, Tr::IN, f.nn);
+  set(Tr::IN, Tr::IBG, f.n);
+  set(Tr::IBG, Tr::IBG, f.s);
+  if constexpr (Tr::EXTRA != 0) {
+    const T ex = Tr::EXTRA == 3 ? wd.dsx * kx.cs() : kx.cs();
+    const T ey = Tr::EXTRA == 3 ? wd.dsy * ky.cs() : ky.cs();
+    const T xa = kx.c * ex * f.xw, xb = kx.c * ey * f.xz, ya = ky.c * ex * f.wy, yb = ky.c * ey * f.ryw;
+    const T na = ex * f.nw, nb = ey * f.rnw, ba = ex * f.w, bb = ey * f.rw;
+    const T aa = ex * ex * f.ww, ab = ex * ey * f.wz, bb2 = ey * ey * f.rww;
+    if constexpr (Tr::EXTRA == 2) {
+      set(Tr::IX, Tr::IE1, xa);
+      set(Tr::IX, Tr::IE2, xb);
+      set(Tr::IY, Tr::IE1, ya);
+      set(Tr::IY, Tr::IE2, yb);
+      set(Tr::IN, Tr::IE1, na);
+      set(Tr::IN, Tr::IE2, nb);
+      set(Tr::IBG, Tr::IE1, ba);
+      set(Tr::IBG, Tr::IE2, bb);
+      set(Tr::IE1, Tr::IE1, aa);
+      set(Tr::IE1, Tr::IE2, ab);
+      set(Tr::IE2, Tr::IE2, bb2);
+    } else {
+      set(Tr::IX, Tr::IE1, xa + xb);
+      set(Tr::IY, Tr::IE1, ya + yb);
+      set(Tr::IN, Tr::IE1, na + nb);
+      set(Tr::IBG, Tr::IE1, ba + bb);
+      set(Tr::IE1, Tr::IE1, aa + T(2) * ab + bb2);
+    }
+  }
+}
+
+// The Fisher sums of columns [c0, c0 + ncol) pixel by pixel, leaving out the
+// pixels whose model is not > 0, as unified_kernel.jl:378-396 does.  The sums
+// above give such pixels weight 0 instead, which a non-finite derivative
+// (non-finite parameters, a width of 0) turns into NaN: an ROI whose matrix is
+// not finite is done again here.  Rolled loops: rare, and small.
+template <int MODEL, int CAM, int N, class T>
+__device__ __forceinline__ void fisher_by_pixel(const T* th, const AxisK<T>& kx, const AxisK<T>& ky,
+                                                const Widths<T>& wd, int c0, int ncol, const float* var, int ny,
+                                                T* Fu) {
+  using Tr = MT<MODEL>;
+  constexpr int P = Tr::P;
+  constexpr bool SIG = Tr::EXTRA != 0;
+#pragma unroll
+  for (int q = 0; q < P * (P + 1) / 2; ++q) Fu[q] = T(0);
+#pragma unroll 1
+  for (int cc = 0; cc < ncol; ++cc) {
+    const T fc = (T)(c0 + cc);
+    const Band<T> cx = band_from_edges<T, SIG>(edge_at<T, SIG>(kx, fc + T(0.5)), edge_at<T, SIG>(kx, fc + T(1.5)));
+#pragma unroll 1
+    for (int i = 0; i < N; ++i) {
+      const Band<T> ry = band_from_edges<T, SIG>(edge_at<T, SIG>(ky, (T)i + T(0.5)), edge_at<T, SIG>(ky, (T)i + T(1.5)));
+      const T mu = th[Tr::IBG] + th[Tr::IN] * cx.phi * ry.phi;
+      if (mu > T(0)) {
+        T wv = T(1) / mu;
+        if constexpr (CAM == SCMOS) wv = T(1) / (mu + (T)var[(int64_t)(c0 + cc) * ny + i]);
+        T du[P];
+        du[Tr::IX] = kx.c * cx.dg * ry.phi;
+        du[Tr::IY] = ky.c * ry.dg * cx.phi;
+        du[Tr::IN] = cx.phi * ry.phi;
+        du[Tr::IBG] = T(1);
+        if constexpr (SIG) {
+          const T ax = (Tr::EXTRA == 3 ? wd.dsx * kx.cs() : kx.cs()) * cx.w;
+          const T ay = (Tr::EXTRA == 3 ? wd.dsy * ky.cs() : ky.cs()) * ry.w;
+          if constexpr (Tr::EXTRA == 2) {
+            du[Tr::IE1] = ax * ry.phi;
+            du[Tr::IE2] = ay * cx.phi;
+          } else {
+            du[Tr::IE1] = ax * ry.phi + ay * cx.phi;
+          }
+        }
+        int q = 0;
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+          const T ak = du[k] * wv;
+#pragma unroll
+          for (int l = k; l < P; ++l) Fu[q++] += ak * du[l];
+        }
+      }
+    }
+  }
+}
+
+// Group sums of the Fisher entries and the LLR, with the pixel-by-pixel matrix
+// where the summed one is not finite (every lane of an ROI takes the same
+// turn: the group sums are the same on all of them).
+template <int MODEL, int CAM, int N, int L, class T>
+__device__ __forceinline__ FinalOut<T, MT<MODEL>::P> final_solve(const T* th, const AxisK<T>& kx, const AxisK<T>& ky,
+                                                               const Widths<T>& wd, T* Fu, T llr, int c0, int ncol,
+                                                               const float* var, int ny) {
+  constexpr int P = MT<MODEL>::P;
+  constexpr int NF = P * (P + 1) / 2;
+  bool fin = true;
+#pragma unroll
+  for (int q = 0; q < NF; ++q) {
+    Fu[q] = group_sum<L>(Fu[q]);
+    fin = fin && (Fu[q] - Fu[q] == T(0));
+  }
+  llr = group_sum<L>(llr);
+  if (__builtin_amdgcn_ballot_w64(!fin) != 0) {
+    T Fp[NF];
+    fisher_by_pixel<MODEL, CAM, N, T>(th, kx, ky, wd, c0, fin ? 0 : ncol, var, ny, Fp);
+#pragma unroll
+    for (int q = 0; q < NF; ++q) {
+      const T f = group_sum<L>(Fp[q]);
+      Fu[q] = fin ? Fu[q] : f;
+    }
+  }
+  FinalOut<T, P> out;
+  out.llr = llr;
+  T F[P * P];
+  int q = 0;
+#pragma unroll
+  for (int k = 0; k < P; ++k)
+#pragma unroll
+    for (int l = k; l < P; ++l) {
+      F[k + P * l] = Fu[q];
+      F[l + P * k] = Fu[q];
+      ++q;
+    }
+  invert_fisher<P, T>(F, out.crlb);
+  return out;
+}
+
+// The Float32 final pass at the estimate th over this lane's register-resident
+// pixels, rows outer and the row values shared as in accumulate().
+template <int MODEL, int CAM, int N, int L>
+__device__ __forceinline__ FinalOut<float, MT<MODEL>::P> final_pass_f32(const float* th, const float* psf, int c0,
+                                                                      int r, const float* dv, const float* vr,
+                                                                      const float* dt, const float* vt, float* roi,
+                                                                      const float* var, int ny) {
+  using Tr = MT<MODEL>;
+  constexpr int P = Tr::P;
+  constexpr bool TAIL = tail_split<N, L>();
+  constexpr int CB = block_cols<N, L>();
+  constexpr int RS = row_slots<N, L>();
+  constexpr bool SIG = Tr::EXTRA != 0;
+  Widths<float> wd;
+  model_widths<MODEL, float>(th, psf, wd);
+  const float nph = th[Tr::IN], bg = th[Tr::IBG];
+  const AxisK<float> kx = axis_consts<float>(th[Tr::IX], wd.sx, nph);
+  const AxisK<float> ky = axis_consts<float>(th[Tr::IY], wd.sy, nph);
+  publish_rows<MODEL, N, L>(ky, r, roi);
+  Band<float> cb[CB], tl{};
+  column_bands<N, L, SIG>(kx, c0, cb, tl);
+  float C[CB], CC[CB], Y[CB], Z[CB];
+#pragma unroll
+  for (int cc = 0; cc < CB; ++cc) C[cc] = CC[cc] = Y[cc] = Z[cc] = 0.f;
+  FisherSums<float> f;
+  float llr = 0.f;
+  if constexpr (TAIL) {
+    float Ct = 0.f, CCt = 0.f, Yt = 0.f, Zt = 0.f;
+#pragma unroll
+    for (int s = 0; s < RS; ++s) {
+      const RowVals v = read_row<MODEL, L>(roi, r * RS + s);
+      const Band<float> b{v.phi, v.dg, v.w, 0.f};
+      const float mu = fmaf(nph * tl.phi, b.phi, bg);
+      float lp, wv;
+      final_weights<CAM, float>(dt[s], CAM == SCMOS ? vt[s] : 0.f, mu, lp, wv);
+      if ((L - 1) * RS + s >= N) {
+        const bool ok = r * RS + s < N;
+        lp = ok ? lp : 0.f;
+        wv = ok ? wv : 0.f;
+      }
+      llr += lp;
+      const float pw = b.phi * wv, xw = tl.phi * wv;
+      Ct += pw;
+      CCt = fmaf(b.phi, pw, CCt);
+      Yt = fmaf(b.dg, pw, Yt);
+      if constexpr (SIG) Zt = fmaf(b.w, pw, Zt);
+      f.s += wv;
+      f.row<SIG>(b, xw, tl.phi * xw);
+    }
+    f.column<SIG>(tl, Ct, CCt, Yt, Zt);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_barrier(0);   // as in accumulate()
+    const RowVals v = read_row<MODEL, L>(roi, i);
+    const Band<float> b{v.phi, v.dg, v.w, 0.f};
+    const float pn = nph * b.phi;
+    float R = 0.f, RR = 0.f;
+#pragma unroll
+    for (int cc = 0; cc < CB; ++cc) {
+      const float mu = fmaf(cb[cc].phi, pn, bg);
+      float lp, wv;
+      final_weights<CAM, float>(dv[cc * N + i], CAM == SCMOS ? vr[cc * N + i] : 0.f, mu, lp, wv);
+      if (may_pad<N, L>(cc)) {
+        lp = c0 + cc < N ? lp : 0.f;
+        wv = c0 + cc < N ? wv : 0.f;
+      }
+      llr += lp;
+      const float pw = b.phi * wv, xw = cb[cc].phi * wv;
+      C[cc] += pw;
+      CC[cc] = fmaf(b.phi, pw, CC[cc]);
+      Y[cc] = fmaf(b.dg, pw, Y[cc]);
+      if constexpr (SIG) Z[cc] = fmaf(b.w, pw, Z[cc]);
+      R += xw;
+      RR = fmaf(cb[cc].phi, xw, RR);
+      f.s += wv;
+    }
+    f.row<SIG>(b, R, RR);
+#pragma unroll
+    for (int cc = 0; cc < CB; ++cc) {
+      asm volatile("" : "+v"(C[cc]), "+v"(CC[cc]), "+v"(Y[cc]));
+      if constexpr (SIG) asm volatile("" : "+v"(Z[cc]));
+    }
+    asm volatile("" : "+v"(f.ry), "+v"(f.ryy), "+v"(f.ryn), "+v"(f.s), "+v"(llr));
+  }
+#pragma unroll
+  for (int cc = 0; cc < CB; ++cc) f.column<SIG>(cb[cc], C[cc], CC[cc], Y[cc], Z[cc]);
+  float Fu[P * (P + 1) / 2];
+  fisher_entries<MODEL, float>(f, kx, ky, wd, Fu);
+  // columns of this lane; the last lane takes the tail column whole
+  int ncol = N - c0 < CB ? (N - c0 < 0 ? 0 : N - c0) : CB;
+  if (TAIL && r == L - 1) ncol = CB + 1;
+  if (CAM == SCMOS && var == nullptr) ncol = 0;   // outside the variance map: nothing to read
+  return final_solve<MODEL, CAM, N, L, float>(th, kx, ky, wd, Fu, llr, c0, ncol, var, ny);
+}
+
 // Out-of-range sCMOS corner: no fit, NaN outputs.
 template <class TF, int P> __device__ __forceinline__ void nan_outputs(float* th, FinalOut<TF, P>& fo) {
   const float qnan = __builtin_nanf("");
@@ -1076,14 +1311,18 @@ struct RoiRef {
 // columns [r*CB, r*CB + CB)).  Every lane of the wave must call this (the
 // cross-lane sums use DPP); `active` lanes store the results.
 template <int MODEL, int CAM, int N, int L, int PREC>
-__device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, bool active, int r) {
+__device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, bool active, int r, float* lds) {
   using Tr = MT<MODEL>;
   constexpr int P = Tr::P;
-  constexpr bool TAIL = tail_split<MODEL, CAM, N, L>();
-  constexpr int CB = block_cols<MODEL, CAM, N, L>();   // full columns per lane
+  constexpr bool TAIL = tail_split<N, L>();
+  constexpr int CB = block_cols<N, L>();   // full columns per lane
   constexpr int RS = row_slots<N, L>();                 // tail split: rows of the last column per lane
   constexpr bool SIG = Tr::EXTRA != 0;  // sigma / z terms present
   const int c0 = r * CB;
+  // this ROI's row values (publish_rows)
+  const int lane = threadIdx.x & (kWave - 1);
+  float* roi = L == 1 ? lds + 4 * lane : lds + lane / L * roi_words<MODEL, N, L>();
+  float* park = lds + rows_words<MODEL, N, L>() + (SIG ? 4 : 2) * lane;   // its columns' (park_band)
 
   // ---- load this lane's column block (and variances) once ----------------
   float dv[CB * N];
@@ -1116,19 +1355,21 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
       if (valid && inb) {
         load_run<N>(a.var_map + (int64_t)(cyc - 1) + (int64_t)a.ny * (int64_t)(cxc - 1 + col), vr + cc * N);
       } else {
+        // an infinite variance gives a padding column's pixels weight 0
+        const float fill = valid ? 0.f : __builtin_inff();
 #pragma unroll
-        for (int i = 0; i < N; ++i) vr[cc * N + i] = 0.f;
+        for (int i = 0; i < N; ++i) vr[cc * N + i] = fill;
       }
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) dmax_l = fmaxf(dmax_l, dv[cc * N + i]);
   }
   if constexpr (TAIL) {
-    // rows r + L s of the last column; slots past the last row hold zeros
-    // (the row index is clamped, so no load leaves the ROI)
+    // rows [r RS, r RS + RS) of the last column; slots past the last row hold
+    // zeros (the row index is clamped, so no load leaves the ROI)
 #pragma unroll
     for (int s = 0; s < RS; ++s) {
-      const int ri = r + L * s;
+      const int ri = r * RS + s;
       const bool ok = ri < N;
       const int rc = ok ? ri : N - 1;
       const float x = src[(N - 1) * N + rc];
@@ -1181,7 +1422,7 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
     if constexpr (TAIL) {
 #pragma unroll
       for (int s = 0; s < RS; ++s) {
-        const int ri = r + L * s;
+        const int ri = r * RS + s;
         const float v = ri < N ? fmaxf(0.f, dt[s] - bg0) : 0.f;
         tot += v;
         xw += v * (float)N;
@@ -1205,13 +1446,15 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
     if constexpr (MODEL == XYNBSXSY) { th[4] = 1.3f; th[5] = 1.3f; }
     if constexpr (MODEL == ASTIG) {
       float mxx = 0.f, myy = 0.f;
+      float b0 = bg0;   // s again from the pixel, instead of every pixel's s kept from above
+      asm volatile("" : "+v"(b0));
 #pragma unroll
       for (int cc = 0; cc < CB; ++cc) {
         const bool valid = (L == 1) || TAIL || (c0 + cc < N);
         const float dxp = (float)(c0 + cc + 1) - x0;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-          const float s = valid ? fmaxf(0.f, dv[cc * N + i] - bg0) : 0.f;
+          const float s = valid ? fmaxf(0.f, dv[cc * N + i] - b0) : 0.f;
           const float dyp = (float)(i + 1) - y0;
           mxx += s * dxp * dxp;
           myy += s * dyp * dyp;
@@ -1221,8 +1464,8 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
         const float dxp = (float)N - x0;
 #pragma unroll
         for (int s = 0; s < RS; ++s) {
-          const int ri = r + L * s;
-          const float v = ri < N ? fmaxf(0.f, dt[s] - bg0) : 0.f;
+          const int ri = r * RS + s;
+          const float v = ri < N ? fmaxf(0.f, dt[s] - b0) : 0.f;
           const float dyp = (float)(ri + 1) - y0;
           mxx += v * dxp * dxp;
           myy += v * dyp * dyp;
@@ -1264,100 +1507,13 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
     }
 
     float G[P], H[P];
-    const AxisK<float> kr = axis_consts<float>(th[Tr::IY], w.sy, nph);
-    constexpr bool SHARE = share_rows<MODEL, CAM, N, L>();
-    if constexpr (row_outer<MODEL, CAM, N, L>()) {
-      const AxisK<float> kc = axis_consts<float>(th[Tr::IX], w.sx, nph);
-      if (fast) {
-        accumulate_rows<MODEL, CAM, N, L, true, SHARE>(dv, vr, dt, vt, c0, nph, bg, kr, r, kc, w, G, H);
-      } else {
-        accumulate_rows<MODEL, CAM, N, L, false, SHARE>(dv, vr, dt, vt, c0, nph, bg, kr, r, kc, w, G, H);
-      }
+    const AxisK<float> kx = axis_consts<float>(th[Tr::IX], w.sx, nph);
+    const AxisK<float> ky = axis_consts<float>(th[Tr::IY], w.sy, nph);
+    publish_rows<MODEL, N, L>(ky, r, roi);
+    if (fast) {
+      accumulate<MODEL, CAM, N, L, true>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, w, roi, park, G, H);
     } else {
-      if constexpr (L == 1) __builtin_amdgcn_s_setprio(0);   // tables and pixel sums: normal priority
-      AxisTab<float, N> ry;
-      const AxisK<float> kc = axis_consts<float>(th[Tr::IX], w.sx, nph);
-      // tail split: the last column's rows r + L s, with this lane's own row
-      // tables, folded here into Gt / Ht
-      float Gt[P], Ht[P];
-#pragma unroll
-      for (int k = 0; k < P; ++k) { Gt[k] = 0.f; Ht[k] = 0.f; }
-      if constexpr (SHARE) {
-        Pix<float> own[RS];
-        shared_axis_tables<N, L, SIG>(kr, r, ry, own);
-        if constexpr (TAIL) {
-          const Pix<float> tl = pix_from_edges<float, SIG>(kc, edge_eval<float, SIG>(kc, N - 1),
-                                                           edge_eval<float, SIG>(kc, N));
-          const float ncx_t = nph * tl.phi;
-          float St[11], rs[6];
-#pragma unroll
-          for (int q = 0; q < 11; ++q) St[q] = 0.f;
-#pragma unroll
-          for (int q = 0; q < 6; ++q) rs[q] = 0.f;
-          if (fast) {
-#pragma unroll
-            for (int s = 0; s < RS; ++s)
-              tail_pixel<MODEL, CAM, true>(own[s], w, dt[s], CAM == SCMOS ? vt[s] : 0.f, r + L * s < N, ncx_t, bg,
-                                           St, rs);
-            tail_fold<MODEL, CAM, true>(St, rs, tl, w, Gt, Ht);
-          } else {
-#pragma unroll
-            for (int s = 0; s < RS; ++s)
-              tail_pixel<MODEL, CAM, false>(own[s], w, dt[s], CAM == SCMOS ? vt[s] : 0.f, r + L * s < N, ncx_t, bg,
-                                            St, rs);
-            tail_fold<MODEL, CAM, false>(St, rs, tl, w, Gt, Ht);
-          }
-        }
-      } else {
-        axis_tables<float, N, SIG>(th[Tr::IY], w.sy, nph, 0, ry);
-      }
-
-      // Row extras: A = d(model)/d(extra) on the row axis, AA its second derivative.
-      float Ay[SIG ? N : 1], AAy[SIG ? N : 1];
-      if constexpr (SIG) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          if constexpr (MODEL == ASTIG) {
-            Ay[i] = w.dsy * ry.S[i];
-            AAy[i] = ry.SS[i] * (w.dsy * w.dsy) + ry.S[i] * w.d2sy;
-          } else {
-            Ay[i] = ry.S[i];
-            AAy[i] = ry.SS[i];
-          }
-        }
-      }
-
-      // Row sums for the q = cf + 1 form of the fast path.
-      float sphi = 0.f, sD = 0.f, sD2 = 0.f, sA = 0.f, sAA = 0.f;
-      if (fast) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          sphi += ry.phi[i];
-          sD += ry.D[i];
-          sD2 += ry.D2[i];
-          if constexpr (SIG) { sA += Ay[i]; sAA += AAy[i]; }
-        }
-      }
-
-      // One lane per ROI: the edge tables and pixel sums run at the normal
-      // wave priority, and the short dependent chain between them (the Newton
-      // step, then the next iteration's widths and axis constants) at a
-      // raised one, so that the SIMD's other wave fills that chain's stalls
-      // with its own pixel work.  (gfx950, XYNB 11 px, 1M ROIs: 1.403 ->
-      // 1.374 ms per launch; raising the tables too gave 1.393, raising the
-      // pixel sums instead 1.431.)  Setting priority 0 again here as well
-      // keeps the compiler's scheduling regions as measured.
-      if constexpr (L == 1) __builtin_amdgcn_s_setprio(0);
-      if (fast) {
-        accumulate<MODEL, CAM, N, L, true>(dv, vr, c0, nph, bg, ry, kc, w, Ay, AAy, sphi, sD, sD2, sA, sAA, G, H);
-      } else {
-        accumulate<MODEL, CAM, N, L, false>(dv, vr, c0, nph, bg, ry, kc, w, Ay, AAy, sphi, sD, sD2, sA, sAA, G, H);
-      }
-      if constexpr (L == 1) __builtin_amdgcn_s_setprio(1);
-      if constexpr (TAIL) {
-#pragma unroll
-        for (int k = 0; k < P; ++k) { G[k] += Gt[k]; H[k] += Ht[k]; }
-      }
+      accumulate<MODEL, CAM, N, L, false>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, w, roi, park, G, H);
     }
 #pragma unroll
     for (int k = 0; k < P; ++k) {
@@ -1391,19 +1547,17 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
     }
   }
 
-  if constexpr (L == 1) __builtin_amdgcn_s_setprio(0);
   // ---- final pass: LLR + Fisher + CRLB (unified_kernel.jl:353-433) --------
   // Float32 here; the Float64 final pass runs as its own kernel
   // (final_pass_kernel) so that its registers do not lower this kernel's
   // occupancy.
   if constexpr (PREC == PREC_FP32) {
-    const RegSrc<N, CAM == SCMOS> srcr{dv, vr, dt, vt};
-    FinalOut<float, P> fo;
-    if constexpr (N > kMaxSmallBox) {
-      fo = final_pass_rows<MODEL, CAM, N, L, float>(th, a.psf, c0, srcr);
-    } else {
-      fo = final_pass<MODEL, CAM, N, L, float, RegSrc<N, CAM == SCMOS>, TAIL>(th, a.psf, c0, srcr, r);
+    const float* var = nullptr;   // the ROI's corner of the variance map
+    if constexpr (CAM == SCMOS) {
+      if (inb) var = a.var_map + (int64_t)(cyc - 1) + (int64_t)a.ny * (int64_t)(cxc - 1);
     }
+    FinalOut<float, P> fo =
+        final_pass_f32<MODEL, CAM, N, L>(th, a.psf, c0, r, dv, vr, dt, vt, roi, var, a.ny);
     if (!inb) nan_outputs(th, fo);
     if (active && r == 0) store_outputs<P>(a, ref.out, ref.stride, th, fo);
   } else {
@@ -1446,7 +1600,8 @@ __device__ __forceinline__ bool locate_roi(const FitArgs& a, int64_t j, int64_t 
 // One launch over n ROIs of one shape: 64/L ROIs per wave, in wave-sized
 // tiles (a grid smaller than the tile count strides over the rest).
 template <int MODEL, int CAM, int N, int L, int PREC>
-__global__ __launch_bounds__(kWave) void fit_kernel(FitArgs a) {
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(min_waves<MODEL, CAM, N, L>())))
+void fit_kernel(FitArgs a) {
   constexpr int RPW = kWave / L;
   const int lane = threadIdx.x;
   const int r = (L == 1) ? 0 : (lane & (L - 1));
@@ -1455,7 +1610,7 @@ __global__ __launch_bounds__(kWave) void fit_kernel(FitArgs a) {
   for (int64_t base = (int64_t)blockIdx.x * RPW; base < a.n_rois; base += (int64_t)gridDim.x * RPW) {
     RoiRef ref;
     const bool active = locate_roi<MODEL, CAM, N>(a, base + lane / L, 0, ref);
-    fit_one<MODEL, CAM, N, L, PREC>(a, ref, active, r);
+    fit_one<MODEL, CAM, N, L, PREC>(a, ref, active, r, wave_lds<wave_words<MODEL, CAM, N, L>()>());
   }
 }
 

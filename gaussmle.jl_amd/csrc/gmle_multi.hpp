@@ -32,6 +32,28 @@ __host__ __device__ constexpr int multi_lanes(int model, int camera, int box, in
   return multi_has(model, camera, box, want) ? want : 4;
 }
 
+// LDS words of the largest tile: every tile function names the same array.
+template <int MODEL, int CAM, int N, int L> constexpr int multi_words_of() {
+  return multi_has(MODEL, CAM, N, L) ? wave_words<MODEL, CAM, N, L>() : 0;
+}
+constexpr int imax(int a, int b) { return a > b ? a : b; }
+template <int MODEL, int CAM, int N> constexpr int multi_words_box() {
+  return imax(multi_words_of<MODEL, CAM, N, 1>(),
+              imax(imax(multi_words_of<MODEL, CAM, N, 2>(), multi_words_of<MODEL, CAM, N, 4>()),
+                   imax(multi_words_of<MODEL, CAM, N, 8>(), multi_words_of<MODEL, CAM, N, 16>())));
+}
+template <int MODEL, int CAM, int N = kMaxBatchBox> constexpr int multi_words_model() {
+  if constexpr (N < kMinBox) {
+    return 0;
+  } else {
+    return imax(multi_words_box<MODEL, CAM, N>(), multi_words_model<MODEL, CAM, N - 1>());
+  }
+}
+template <int CAM> constexpr int multi_words() {
+  return imax(imax(multi_words_model<XYNB, CAM>(), multi_words_model<XYNBS, CAM>()),
+              imax(multi_words_model<XYNBSXSY, CAM>(), multi_words_model<ASTIG, CAM>()));
+}
+
 struct MultiArgs {
   FitArgs fa[4];                  // per model: psf / constraints; shared data, order and outputs
   int32_t n_entries;
@@ -67,7 +89,7 @@ __device__ __attribute__((noinline)) void multi_tile(const FitArgs& a, int32_t f
     ref.cx = a.x_corners[k];
     ref.cy = a.y_corners[k];
   }
-  fit_one<MODEL, CAM, N, L, PREC_FP32>(a, ref, active, r);
+  fit_one<MODEL, CAM, N, L, PREC_FP32>(a, ref, active, r, wave_lds<multi_words<CAM>()>());
 }
 
 template <int CAM, int MODEL, int N>
