@@ -455,18 +455,18 @@ __device__ __forceinline__ void model_widths(const T* th, const float* psf, Widt
 // One pixel's likelihood weights (camera_models.jl:19-42): cf multiplies the
 // model's derivatives in the gradient, df in the Hessian.  FAST (Poisson
 // only): every model value exceeds 0.01 and neither 1e4 cap can bind; then
-// cf = d/mu - 1 and df = d/mu^2 = (cf + 1)/mu are one FMA each.
+// cf = d/mu - 1 and df = d/mu^2 = (cf + 1)/mu are one FMA each.  Where no mask
+// binds both forms give the same bits.
 template <int CAM, bool FAST>
 __device__ __forceinline__ void pixel_weights(float d, float var, float mu, float& cf, float& df) {
   if constexpr (CAM == IDEAL) {
     const float rc = fast_rcp(mu);
+    const float a = fmaf(d, rc, -1.f), b = fmaf(a, rc, rc);
     if constexpr (FAST) {
-      cf = fmaf(d, rc, -1.f);
-      df = fmaf(cf, rc, rc);
+      cf = a;
+      df = b;
     } else {
-      const float q = d * rc;
       const bool pos = mu > 0.01f;   // camera_models.jl:23-32
-      const float a = q - 1.f, b = q * rc;
       cf = pos ? (1.0e4f < a ? 1.0e4f : a) : 0.f;   // Julia's min: a NaN passes
       df = pos ? (1.0e4f < b ? 1.0e4f : b) : 0.f;
     }
@@ -519,13 +519,18 @@ __device__ __forceinline__ void column_bands(const AxisK<float>& kx, int c0, Ban
 // Bound by VALU issue.  gfx950, ms per launch against 7 to 11 sums per pixel
 // with the row tables by DPP: sCMOS XYNBS 13 px, 1M ROIs 3.20 -> 2.36; astigmatic
 // 15 px, 1M 6.07 -> 3.96; XYNBS 21 px, 200K 1.80 -> 1.02; XYNB 11 px on one lane,
-// 1M 1.386 -> 1.369.
+// 1M 1.386 -> 1.369 (on two lanes, the default at that size, 1.254).
 // ---------------------------------------------------------------------------
+struct PixelSums {
+  float a1, a2, a3, a4, a5;   // columns: dg C, w C, dg^2 CC, t3 C, w^2 CC
+  float y1, y2, y3, y4, y5;   // rows: dg R, w R, t3 R, dg^2 RR, w^2 RR
+  float gn, hn, xs;           // phi C, phi^2 CC, phi w X
+  float scf, sdf;
+};
 template <int MODEL, int CAM, int N, int L, bool FAST>
 __device__ __forceinline__ void accumulate(const float* dv, const float* vr, const float* dt, const float* vt, int c0,
                                            int r, float nph, float bg, const AxisK<float>& kx, const AxisK<float>& ky,
-                                           const Widths<float>& w, const float* roi, float* park, float* G,
-                                           float* H) {
+                                           const float* roi, float* park, PixelSums& out) {
   using Tr = MT<MODEL>;
   constexpr bool TAIL = tail_split<N, L>();
   constexpr int CB = block_cols<N, L>();
@@ -657,20 +662,30 @@ __device__ __forceinline__ void accumulate(const float* dv, const float* vr, con
       sdf += c0 + cc < N ? pad_df[cc] : 0.f;
     }
   }
-  G[Tr::IX] = kx.c * a1;
-  H[Tr::IX] = kx.c2() * a2 - (kx.c * kx.c) * a3;
-  G[Tr::IY] = ky.c * y1;
-  H[Tr::IY] = ky.c2() * y2 - (ky.c * ky.c) * y4;
-  G[Tr::IN] = gn;
-  H[Tr::IN] = -hn;
-  G[Tr::IBG] = scf;
-  H[Tr::IBG] = -sdf;
+  out = PixelSums{a1, a2, a3, a4, a5, y1, y2, y3, y4, y5, gn, hn, xs, scf, sdf};
+}
+
+// The gradient and diagonal Hessian from the sums: once for both forms of the
+// pixel loop, so that an ROI's result does not depend on which one its wave took.
+template <int MODEL>
+__device__ __forceinline__ void gradient(const PixelSums& u, const AxisK<float>& kx, const AxisK<float>& ky,
+                                         const Widths<float>& w, float* G, float* H) {
+  using Tr = MT<MODEL>;
+  constexpr bool SIG = Tr::EXTRA != 0;
+  G[Tr::IX] = kx.c * u.a1;
+  H[Tr::IX] = kx.c2() * u.a2 - (kx.c * kx.c) * u.a3;
+  G[Tr::IY] = ky.c * u.y1;
+  H[Tr::IY] = ky.c2() * u.y2 - (ky.c * ky.c) * u.y4;
+  G[Tr::IN] = u.gn;
+  H[Tr::IN] = -u.hn;
+  G[Tr::IBG] = u.scf;
+  H[Tr::IBG] = -u.sdf;
   if constexpr (SIG) {
     // width terms of each axis: first derivative ex w, second (m2s + d2) w + css t3
-    const float csx = kx.cs() * a2, csy = ky.cs() * y2;                       // sum S C, sum S R
-    const float ssx = kx.m2s() * csx + kx.css() * a4, ssy = ky.m2s() * csy + ky.css() * y3;   // sum SS C, sum SS R
-    const float qx = kx.cs() * kx.cs() * a5, qy = ky.cs() * ky.cs() * y5;         // sum S^2 CC, sum S^2 RR
-    const float qxy = 2.f * (kx.cs() * ky.cs()) * xs;
+    const float csx = kx.cs() * u.a2, csy = ky.cs() * u.y2;                       // sum S C, sum S R
+    const float ssx = kx.m2s() * csx + kx.css() * u.a4, ssy = ky.m2s() * csy + ky.css() * u.y3;   // sum SS C, sum SS R
+    const float qx = kx.cs() * kx.cs() * u.a5, qy = ky.cs() * ky.cs() * u.y5;         // sum S^2 CC, sum S^2 RR
+    const float qxy = 2.f * (kx.cs() * ky.cs()) * u.xs;
     if constexpr (MODEL == XYNBS) {
       G[Tr::IE1] = csx + csy;
       H[Tr::IE1] = ssx + ssy - qx - qy - qxy;
@@ -1510,11 +1525,16 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
     const AxisK<float> kx = axis_consts<float>(th[Tr::IX], w.sx, nph);
     const AxisK<float> ky = axis_consts<float>(th[Tr::IY], w.sy, nph);
     publish_rows<MODEL, N, L>(ky, r, roi);
-    if (fast) {
-      accumulate<MODEL, CAM, N, L, true>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, w, roi, park, G, H);
+    // One form for the whole wave: where some ROI needs the masks, running both
+    // in turn would cost the others' pixel loop again (XYNB 11 px, backgrounds
+    // of 1-20 photons: 1.271 -> 1.254 ms per 1M ROIs, 40.9 -> 39.7 us per 10,000).
+    PixelSums u;
+    if (__builtin_amdgcn_ballot_w64(CAM == IDEAL && !fast) == 0) {
+      accumulate<MODEL, CAM, N, L, true>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, roi, park, u);
     } else {
-      accumulate<MODEL, CAM, N, L, false>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, w, roi, park, G, H);
+      accumulate<MODEL, CAM, N, L, false>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, roi, park, u);
     }
+    gradient<MODEL>(u, kx, ky, w, G, H);
 #pragma unroll
     for (int k = 0; k < P; ++k) {
       G[k] = group_sum<L>(G[k]);
