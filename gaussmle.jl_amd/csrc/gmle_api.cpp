@@ -103,16 +103,17 @@ bool lanes_ok(int box, int lanes) { return lanes_built(box, lanes); }
 // Lanes per ROI for a large batch.  Fewer lanes repeat less per-ROI work and
 // share fewer rows; more lanes leave a lane fewer pixels, so that three waves
 // per SIMD fit, or two.  Where the lines lie (gfx950, ns per ROI, 1M ROIs):
-//   1 -> 2 lanes  ideal, 7 px 0.69 / 0.72 to 0.79 / 0.86 by model, 9 px 1.04 / 0.95
-//                 to 1.73 / 1.26; sCMOS, 5 px 0.45 / 0.54, 7 px 0.77 / 0.73
+//   1 -> 2 lanes  ideal, 8 px 0.73 / 0.80 to 1.10 / 0.99 by model, 9 px with a
+//                 width 1.26 / 1.14 to 1.76 / 1.24; XYNB 11 px 1.19 / 1.22,
+//                 12 px 1.35 / 1.28; sCMOS, 7 px 0.67 / 0.74 to 0.82 / 0.93,
+//                 8 px equal, 10 px 1.50 / 1.14 to 1.77 / 1.33
 //   2 -> 4 lanes  ideal, 14 px 1.84 / 2.12 to 2.22 / 2.65, 16 px 2.21 / 2.25 to
 //                 2.82 / 2.80; sCMOS, 11 px 1.39 / 1.54 to 1.77 / 1.93, 13 px
 //                 2.50 / 1.97 to 3.12 / 2.84
-// XYNB with an ideal camera keeps one lane up to 11 px here (default_lanes).
 int large_batch_lanes(int model, int camera, int box) {
   if (box > kMaxSmallBox) return large_box_lanes(model, camera, box);
   const bool sc = camera == SCMOS;
-  const int one = sc ? 6 : model == XYNB ? 11 : 7, two = sc ? 12 : 14;
+  const int one = sc ? 7 : model == XYNB ? 11 : 8, two = sc ? 12 : 14;
   return box <= one ? 1 : box <= two ? 2 : 4;
 }
 
@@ -127,10 +128,6 @@ int default_lanes(int model, int camera, int box, int precision, int64_t n_rois)
   const int64_t fill = 256 * 4 * 64;   // CUs x SIMDs x lanes: one wave per SIMD
   int lanes = large_batch_lanes(model, camera, box);
   if (!lanes_ok(box, lanes)) lanes = box > kMaxSmallBox ? 16 : 2;
-  // XYNB 8 to 11 px: two lanes (11 px 1.41 -> 1.24 ns per ROI at 1M ROIs, 1.83 ->
-  // 1.55 at 200K).  Beyond 4M ROIs per call the answer of gmle_default_lanes is
-  // fixed at one lane (tests/test_abi.py), and the sizes above were not timed.
-  if (lanes == 1 && box > 7 && n_rois <= (int64_t)1 << 22) lanes = 2;
   for (int more = 2; more <= 16; more *= 2)
     if (lanes < more && n_rois * more <= fill && lanes_ok(box, more)) lanes = more;
   return lanes;

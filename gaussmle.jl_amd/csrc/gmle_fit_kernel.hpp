@@ -519,7 +519,7 @@ __device__ __forceinline__ void column_bands(const AxisK<float>& kx, int c0, Ban
 // Bound by VALU issue.  gfx950, ms per launch against 7 to 11 sums per pixel
 // with the row tables by DPP: sCMOS XYNBS 13 px, 1M ROIs 3.20 -> 2.36; astigmatic
 // 15 px, 1M 6.07 -> 3.96; XYNBS 21 px, 200K 1.80 -> 1.02; XYNB 11 px on one lane,
-// 1M 1.386 -> 1.369 (on two lanes, the default at that size, 1.254).
+// 1M 1.386 -> 1.144.
 // ---------------------------------------------------------------------------
 struct PixelSums {
   float a1, a2, a3, a4, a5;   // columns: dg C, w C, dg^2 CC, t3 C, w^2 CC
@@ -1161,7 +1161,7 @@ __device__ __forceinline__ FinalOut<T, MT<MODEL>::P> final_solve(const T* th, co
 #pragma unroll
   for (int q = 0; q < NF; ++q) {
     Fu[q] = group_sum<L>(Fu[q]);
-    fin = fin && (Fu[q] - Fu[q] == T(0));
+    fin = fin && __builtin_isfinite(Fu[q]);   // not x - x == 0: x is a product, which contracts into the difference
   }
   llr = group_sum<L>(llr);
   if (__builtin_amdgcn_ballot_w64(!fin) != 0) {
