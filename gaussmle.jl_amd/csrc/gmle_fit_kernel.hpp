@@ -88,8 +88,10 @@ template <> struct DM<float> {
     const float e = fmaf(-b, r, 1.f);
     return fabsf(e) < 1.f ? fmaf(e, r, r) : r;
   }
-  // The scale t -> v of an edge, k / (sigma sqrt 2).
-  static __device__ __forceinline__ float erf_rate(float, float inv_s) { return inv_s * kErfRate; }
+  // The scale t -> v of an edge, k / (|sigma| sqrt 2): the reference's
+  // sqrt(1 / (2 sigma^2)), which a negative width (bounds below 0 allow one)
+  // does not turn round.
+  static __device__ __forceinline__ float erf_rate(float, float inv_s) { return fabsf(inv_s) * kErfRate; }
 };
 template <> struct DM<double> {
   static __device__ __forceinline__ double erf_scale() { return 1.0; }
