@@ -117,6 +117,12 @@ int large_batch_lanes(int model, int camera, int box) {
   return box <= one ? 1 : box <= two ? 2 : 4;
 }
 
+// Lanes of a shape in the multi-shape kernel, `lanes` requested (0: automatic).
+int one_launch_lanes(int model, int camera, int box, int lanes) {
+  return lanes > 0 ? multi_lanes(model, camera, box, lanes)
+                   : multi_auto_lanes(model, camera, box, large_batch_lanes(model, camera, box));
+}
+
 // Lanes per ROI when the caller passes 0: the large-batch choice, raised to
 // the most lanes that keep the launch within one wave per SIMD.  Below that
 // the chip is latency-bound and more, shorter waves finish sooner; above it
@@ -489,10 +495,9 @@ int enqueue_batch(const BatchSpec& b, hipStream_t stream) {
     for (int qm = 0; qm < n_multi; ++qm) {
       const int s = multi[qm];
       const int model = s / kNumBoxes, box = kMinBox + s % kNumBoxes;
-      const int want = (b.lanes && b.lanes[s] > 0) ? b.lanes[s] : large_batch_lanes(model, b.camera, box);
       const int q = m.n_entries++;
       m.shape[q] = s;
-      m.lanes[q] = multi_lanes(model, b.camera, box, want);
+      m.lanes[q] = one_launch_lanes(model, b.camera, box, b.lanes ? b.lanes[s] : 0);
       m.first[q] = p.start[s];
       m.count[q] = p.count[s];
     }
@@ -784,7 +789,7 @@ int gmle_shape_index(int model, int box) { return shape_index(model, box); }
 int gmle_one_launch_lanes(int model, int camera, int box, int lanes) {
   if (shape_index(model, box) < 0 || (camera != IDEAL && camera != SCMOS)) return 0;
   if (!multi_eligible(model, camera, box)) return 0;
-  return multi_lanes(model, camera, box, lanes > 0 ? lanes : large_batch_lanes(model, camera, box));
+  return one_launch_lanes(model, camera, box, lanes);
 }
 
 size_t gmle_batch_workspace_bytes(int64_t n_rois) { return batch_workspace(n_rois < 0 ? 0 : n_rois); }

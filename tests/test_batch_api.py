@@ -186,3 +186,15 @@ def test_one_launch_lanes(hiplib):
     assert hiplib.gmle_one_launch_lanes(1, 0, 16, 8) == 4     # 16 px sigma models: no 8-lane tile within 256
     assert hiplib.gmle_one_launch_lanes(9, 0, 11, 1) == 0
 
+
+def test_one_launch_automatic_lanes(hiplib):
+    """The fewest lanes with a tile, from the large-batch choice on."""
+    for m in range(4):
+        for cam in (0, 1):
+            for b in range(3, 17):
+                auto = hiplib.gmle_one_launch_lanes(m, cam, b, 0)
+                want = hiplib.gmle_default_lanes(m, cam, b, 0, 10**7)
+                if auto:
+                    tiles = [n for n in (1, 2, 4) if n >= want and hiplib.gmle_one_launch_lanes(m, cam, b, n) == n]
+                    assert auto == tiles[0], (m, cam, b, want, tiles)
+
