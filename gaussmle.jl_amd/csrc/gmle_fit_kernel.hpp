@@ -267,7 +267,8 @@ template <bool SIG> __device__ __forceinline__ RowVals row_vals(const Band<float
 // reads a row's values (one or two 16-byte reads at one address per ROI) when
 // its loop reaches the row.  LDS reads issue beside the VALU, where the DPP
 // moves used before took 5 VALU instructions per row at 2 and 4 lanes and 15
-// at 8.  The wave is its own only reader, and LDS operations of a wave stay in
+// at 8 (one per value at 16, where the read's latency counts instead: see
+// rows_together).  The wave is its own only reader, and LDS operations of a wave stay in
 // order, so no barrier is needed beyond the compiler's.  An ROI's rows take
 // RS L slots (slots past row N - 1 are written and never read) plus 4 words,
 // which spread the ROIs that one 16-lane phase of a read serves over the banks.
@@ -296,9 +297,10 @@ __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// This lane's rows, evaluated and written to its ROI's LDS words.
+// This lane's rows, evaluated and written to its ROI's LDS words (and to own,
+// unless null).
 template <int MODEL, int N, int L>
-__device__ __forceinline__ void publish_rows(const AxisK<float>& ky, int r, float* roi) {
+__device__ __forceinline__ void publish_rows(const AxisK<float>& ky, int r, float* roi, RowVals* own = nullptr) {
   constexpr bool SIG = MT<MODEL>::EXTRA != 0;
   constexpr int RS = row_slots<N, L>();
   constexpr int W = row_stride<MODEL, L>();
@@ -311,6 +313,7 @@ __device__ __forceinline__ void publish_rows(const AxisK<float>& ky, int r, floa
     const Edge<float> hi = edge_at<float, SIG>(ky, r0 + ((float)s + 1.5f));
     const RowVals v = row_vals<SIG>(band_from_edges<float, SIG>(lo, hi));
     lo = hi;
+    if (own) own[s] = v;
     float4* q = reinterpret_cast<float4*>(dst + s * W);
     if constexpr (SIG && L > 1) {
       q[0] = make_float4(v.phi, v.phi2, v.pw, v.dg);
@@ -354,12 +357,14 @@ template <int N, int L> constexpr bool tail_split() { return L >= 4 && N > L && 
 template <int N, int L> constexpr int block_cols() {
   return tail_split<N, L>() ? N / L : (N + L - 1) / L;
 }
-// Rows whose pixel work the scheduler may mix: a row of few columns is a short
-// dependent chain (model, reciprocal, weights, sums), so several go together.
-// About four pixels: sCMOS XYNBS 13 px (3 columns) runs 2.30 ms per 1M ROIs one
-// row at a time and 2.36 two rows together; 100 ROIs of 7 px (one column) run
-// 25.0 us one row at a time and 24.3 together.
-template <int CB> constexpr int rows_together() { return CB >= 4 ? 1 : 4 / CB; }
+// Rows whose pixel work the scheduler may mix, and that are read from LDS
+// together, one such group ahead: a row of one column is a short dependent chain
+// (model, reciprocal, weights, sums), so two go together.  us per launch on 16
+// lanes with groups of 1, 2 and 4: sCMOS XYNB 13 px, 2,000 ROIs 24.5, 23.2, 23.2;
+// XYNBSXSY 9 px, 4,000 ROIs 29.0, 28.8, 31.6.  From two columns on, one row at a time
+// (sCMOS XYNBS 13 px, 3 columns, 1M ROIs 2.30 ms, two rows together 2.36;
+// astigmatic 21 px, 2 columns on 16 lanes 59.3 us and 62.0).
+template <int CB> constexpr int rows_together() { return CB == 1 ? 2 : 1; }
 // Least waves per SIMD a fit kernel is built for: three where a lane's pixels (and
 // variances) leave the loop enough of the 168 VGPRs that three waves have, and
 // three waves' LDS fits a CU's 160 KB, else two where a few spilled values
@@ -406,6 +411,30 @@ template <bool SIG> __device__ __forceinline__ Band<float> parked_band(const flo
 // N).  Such a column carries zero column values and adds nothing.
 template <int N, int L> constexpr bool may_pad(int cc) {
   return !tail_split<N, L>() && (L - 1) * block_cols<N, L>() + cc >= N;
+}
+
+// Tail split: whether a lane keeps the values of the rows it evaluated in
+// registers for its pixels of the last column, which then need not wait for LDS.
+// Up to three of them, or under sCMOS: the two forms of the Poisson loop hold
+// more, and four rows spilled there (XYNB 13 px on 4 lanes, 12,000 ROIs: 49.8 us
+// through LDS, 56.2 from registers; sCMOS 51.9 and 50.1).
+template <int CAM, int N, int L> constexpr bool keep_own_rows() {
+  return tail_split<N, L>() && (CAM == SCMOS || row_slots<N, L>() <= 3);
+}
+// Rows 0 .. KR - 1, and in the loop the KR rows from i on while the next KR are
+// in flight.
+template <int MODEL, int N, int L, int KR>
+__device__ __forceinline__ void first_rows(const float* roi, RowVals* next) {
+#pragma unroll
+  for (int k = 0; k < KR; ++k) next[k] = read_row<MODEL, L>(roi, k < N ? k : 0);
+}
+template <int MODEL, int N, int L, int KR>
+__device__ __forceinline__ void take_rows(const float* roi, int i, RowVals* rows, RowVals* next) {
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+    rows[k] = next[k];
+    if (i + KR + k < N) next[k] = read_row<MODEL, L>(roi, i + KR + k);
+  }
 }
 
 // Per-ROI width parameters for one evaluation of the model.
@@ -532,7 +561,7 @@ struct PixelSums {
 template <int MODEL, int CAM, int N, int L, bool FAST>
 __device__ __forceinline__ void accumulate(const float* dv, const float* vr, const float* dt, const float* vt, int c0,
                                            int r, float nph, float bg, const AxisK<float>& kx, const AxisK<float>& ky,
-                                           const float* roi, float* park, PixelSums& out) {
+                                           const float* roi, const RowVals* own, float* park, PixelSums& out) {
   using Tr = MT<MODEL>;
   constexpr bool TAIL = tail_split<N, L>();
   constexpr int CB = block_cols<N, L>();
@@ -540,6 +569,12 @@ __device__ __forceinline__ void accumulate(const float* dv, const float* vr, con
   constexpr bool SIG = Tr::EXTRA != 0;
   constexpr bool TWO = (Tr::EXTRA == 1 || Tr::EXTRA == 3);
   constexpr int KR = rows_together<CB>();
+  // One column: its factor multiplies the row sums once, not every row's cf and
+  // df.  With the rows read ahead in twos and the shorter Newton test below, us per
+  // launch: sCMOS XYNB 13 px, 2,000 ROIs on 16 lanes 27.0 -> 23.2, ideal XYNB 7 px,
+  // 100 ROIs 20.9 -> 19.5, XYNBSXSY 9 px, 4,000 ROIs 30.4 -> 28.8.
+  constexpr bool ONE = CB == 1;
+  constexpr bool OWN = keep_own_rows<CAM, N, L>();
   Band<float> cb[CB], tl{};
   column_bands<N, L, SIG>(kx, c0, cb, tl);
   constexpr bool PARK = park_words<MODEL, CAM, N, L>() != 0;
@@ -588,7 +623,7 @@ __device__ __forceinline__ void accumulate(const float* dv, const float* vr, con
 #pragma unroll
     for (int s = 0; s < RS; ++s) {
       if (s % KR == 0) __builtin_amdgcn_sched_barrier(0);
-      const RowVals v = read_row<MODEL, L>(roi, r * RS + s);
+      const RowVals v = OWN ? own[s] : read_row<MODEL, L>(roi, r * RS + s);
       const float mu = fmaf(npx, v.phi, bg);
       float cf, df;
       pixel_weights<CAM, FAST>(dt[s], CAM == SCMOS ? vt[s] : 0.f, mu, cf, df);
@@ -611,15 +646,18 @@ __device__ __forceinline__ void accumulate(const float* dv, const float* vr, con
     if constexpr (SIG) asm volatile("" : "+v"(a4), "+v"(a5), "+v"(y3), "+v"(y5), "+v"(xs));
     __builtin_amdgcn_sched_barrier(0);
   }
-  // Row i's values are read from LDS during row i - 1.
-  RowVals next = read_row<MODEL, L>(roi, 0);
+  RowVals rows[KR], next[KR];
+  first_rows<MODEL, N, L, KR>(roi, next);
+  float z1 = 0.f, z2 = 0.f, z3 = 0.f, z4 = 0.f, z5 = 0.f;   // ONE: the row sums before their column factor
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     // Keep the rows' work apart: without this the scheduler hoists later rows'
     // values and pixel products and they all become live at once.
-    if (i % KR == 0) __builtin_amdgcn_sched_barrier(0);
-    const RowVals v = next;
-    if (i + 1 < N) next = read_row<MODEL, L>(roi, i + 1);
+    if (i % KR == 0) {
+      __builtin_amdgcn_sched_barrier(0);
+      take_rows<MODEL, N, L, KR>(roi, i, rows, next);
+    }
+    const RowVals v = rows[i % KR];
     const float pn = nph * v.phi;
     float R = 0.f, RR = 0.f;
 #pragma unroll
@@ -630,8 +668,18 @@ __device__ __forceinline__ void accumulate(const float* dv, const float* vr, con
       C[cc] = fmaf(v.phi, cf, C[cc]);
       CC[cc] = fmaf(v.phi2, df, CC[cc]);
       if constexpr (TWO) X[cc] = fmaf(v.pw, df, X[cc]);
-      R = cc == 0 ? cb[cc].phi * cf : fmaf(cb[cc].phi, cf, R);
-      RR = cc == 0 ? px2[cc] * df : fmaf(px2[cc], df, RR);
+      if constexpr (ONE) {
+        z1 = fmaf(v.dg, cf, z1);
+        z2 = fmaf(v.w, cf, z2);
+        z4 = fmaf(v.dg2, df, z4);
+        if constexpr (SIG) {
+          z3 = fmaf(v.t3, cf, z3);
+          z5 = fmaf(v.w2, df, z5);
+        }
+      } else {
+        R = cc == 0 ? cb[cc].phi * cf : fmaf(cb[cc].phi, cf, R);
+        RR = cc == 0 ? px2[cc] * df : fmaf(px2[cc], df, RR);
+      }
       // A padding pixel has data 0; its weights are 0 under sCMOS (infinite
       // variance), and are dropped after the rows for the ideal camera.
       if (CAM == IDEAL && may_pad<N, L>(cc)) {
@@ -642,7 +690,7 @@ __device__ __forceinline__ void accumulate(const float* dv, const float* vr, con
         sdf += df;
       }
     }
-    fold_row(v, R, RR);
+    if constexpr (!ONE) fold_row(v, R, RR);
     // ... and tie this row's sums to the end of the row, or instruction
     // selection sinks the pixel work of every row below the last one.
     if (i % KR != KR - 1) continue;
@@ -652,9 +700,16 @@ __device__ __forceinline__ void accumulate(const float* dv, const float* vr, con
       if constexpr (TWO) asm volatile("" : "+v"(X[cc]));
       if (CAM == IDEAL && may_pad<N, L>(cc)) asm volatile("" : "+v"(pad_cf[cc]), "+v"(pad_df[cc]));
     }
-    asm volatile("" : "+v"(y1), "+v"(y2), "+v"(y4), "+v"(scf), "+v"(sdf));
-    if constexpr (SIG) asm volatile("" : "+v"(y3), "+v"(y5));
+    asm volatile("" : "+v"(scf), "+v"(sdf));
+    if constexpr (ONE) {
+      asm volatile("" : "+v"(z1), "+v"(z2), "+v"(z4));
+      if constexpr (SIG) asm volatile("" : "+v"(z3), "+v"(z5));
+    } else {
+      asm volatile("" : "+v"(y1), "+v"(y2), "+v"(y4));
+      if constexpr (SIG) asm volatile("" : "+v"(y3), "+v"(y5));
+    }
   }
+  if constexpr (ONE) fold_row(RowVals{0.f, 0.f, 0.f, z1, z2, z3, z4, z5}, cb[0].phi, px2[0]);
 #pragma unroll
   for (int cc = 0; cc < CB; ++cc) {
     fold_col(PARK ? parked_band<SIG>(park, cc, cb[cc].phi) : cb[cc], px2[cc], C[cc], CC[cc],
@@ -1209,7 +1264,9 @@ __device__ __forceinline__ FinalOut<float, MT<MODEL>::P> final_pass_f32(const fl
   const float nph = th[Tr::IN], bg = th[Tr::IBG];
   const AxisK<float> kx = axis_consts<float>(th[Tr::IX], wd.sx, nph);
   const AxisK<float> ky = axis_consts<float>(th[Tr::IY], wd.sy, nph);
-  publish_rows<MODEL, N, L>(ky, r, roi);
+  constexpr bool OWN = keep_own_rows<CAM, N, L>();
+  RowVals own[OWN ? RS : 1];
+  publish_rows<MODEL, N, L>(ky, r, roi, OWN ? own : nullptr);
   Band<float> cb[CB], tl{};
   column_bands<N, L, SIG>(kx, c0, cb, tl);
   float C[CB], CC[CB], Y[CB], Z[CB];
@@ -1221,7 +1278,7 @@ __device__ __forceinline__ FinalOut<float, MT<MODEL>::P> final_pass_f32(const fl
     float Ct = 0.f, CCt = 0.f, Yt = 0.f, Zt = 0.f;
 #pragma unroll
     for (int s = 0; s < RS; ++s) {
-      const RowVals v = read_row<MODEL, L>(roi, r * RS + s);
+      const RowVals v = OWN ? own[s] : read_row<MODEL, L>(roi, r * RS + s);
       const Band<float> b{v.phi, v.dg, v.w, 0.f};
       const float mu = fmaf(nph * tl.phi, b.phi, bg);
       float lp, wv;
@@ -1242,10 +1299,12 @@ __device__ __forceinline__ FinalOut<float, MT<MODEL>::P> final_pass_f32(const fl
     }
     f.column<SIG>(tl, Ct, CCt, Yt, Zt);
   }
+  RowVals next = read_row<MODEL, L>(roi, 0);   // with one column per lane, a row ahead
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     __builtin_amdgcn_sched_barrier(0);   // as in accumulate()
-    const RowVals v = read_row<MODEL, L>(roi, i);
+    const RowVals v = CB == 1 ? next : read_row<MODEL, L>(roi, i);
+    if (CB == 1 && i + 1 < N) next = read_row<MODEL, L>(roi, i + 1);
     const Band<float> b{v.phi, v.dg, v.w, 0.f};
     const float pn = nph * b.phi;
     float R = 0.f, RR = 0.f;
@@ -1335,6 +1394,7 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
   constexpr int CB = block_cols<N, L>();   // full columns per lane
   constexpr int RS = row_slots<N, L>();                 // tail split: rows of the last column per lane
   constexpr bool SIG = Tr::EXTRA != 0;  // sigma / z terms present
+  constexpr bool OWN = keep_own_rows<CAM, N, L>();
   const int c0 = r * CB;
   // this ROI's row values (publish_rows)
   const int lane = threadIdx.x & (kWave - 1);
@@ -1526,15 +1586,16 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
     float G[P], H[P];
     const AxisK<float> kx = axis_consts<float>(th[Tr::IX], w.sx, nph);
     const AxisK<float> ky = axis_consts<float>(th[Tr::IY], w.sy, nph);
-    publish_rows<MODEL, N, L>(ky, r, roi);
+    RowVals own[OWN ? RS : 1];
+    publish_rows<MODEL, N, L>(ky, r, roi, OWN ? own : nullptr);
     // One form for the whole wave: where some ROI needs the masks, running both
     // in turn would cost the others' pixel loop again (XYNB 11 px, backgrounds
     // of 1-20 photons: 1.271 -> 1.254 ms per 1M ROIs, 40.9 -> 39.7 us per 10,000).
     PixelSums u;
     if (__builtin_amdgcn_ballot_w64(CAM == IDEAL && !fast) == 0) {
-      accumulate<MODEL, CAM, N, L, true>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, roi, park, u);
+      accumulate<MODEL, CAM, N, L, true>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, roi, own, park, u);
     } else {
-      accumulate<MODEL, CAM, N, L, false>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, roi, park, u);
+      accumulate<MODEL, CAM, N, L, false>(dv, vr, dt, vt, c0, r, nph, bg, kx, ky, roi, own, park, u);
     }
     gradient<MODEL>(u, kx, ky, w, G, H);
 #pragma unroll
@@ -1547,15 +1608,17 @@ __device__ __forceinline__ void fit_one(const FitArgs& a, const RoiRef& ref, boo
     // both are below 1e30 in magnitude; a lane with a NaN, an infinity or a
     // value beyond that takes the IEEE division, so those cases come out as
     // the division gives them.  The division runs only in a wave that has
-    // such a lane.
-    float step[P];
-    bool exact = true;
+    // such a lane.  One sum of the magnitudes is tested: it is NaN, infinite or
+    // large where one of them is, and a test of each became a packed bit mask of
+    // three instructions per value.
+    float step[P], size = 0.f;
 #pragma unroll
     for (int k = 0; k < P; ++k) {
       const float g = G[k], h = H[k];
       step[k] = fabsf(h) > 1e-10f ? g * __builtin_amdgcn_rcpf(h) : 0.f;
-      exact = exact && fabsf(g) < 1e30f && fabsf(h) < 1e30f;
+      size += fabsf(g) + fabsf(h);
     }
+    const bool exact = size < 1e30f;
     if (__builtin_amdgcn_ballot_w64(!exact) != 0) {
 #pragma unroll
       for (int k = 0; k < P; ++k)
