@@ -1055,7 +1055,8 @@ template <int CAM, class T> __device__ __forceinline__ void final_weights(T d, T
     const T v = mu + var;   // camera_models.jl:73-85
     const T res = d - mu;
     const T rv = T(1) / v;
-    lp = v > T(0) ? T(-0.5) * (res * res * rv) : T(0);
+    // the clamp: 1 / v of a denormal v is infinite, and 0 x inf no LLR term
+    lp = v > T(0) ? T(-0.5) * (res * res * fminf(rv, 3.40282347e38f)) : T(0);
     wv = mu > T(0) ? rv : T(0);
   }
 }
