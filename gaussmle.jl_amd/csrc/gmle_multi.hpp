@@ -74,12 +74,22 @@ struct MultiArgs {
   int32_t block_start[kNumShapes + 1];   // first block (= tile) of entry q; total at n_entries
 };
 
+// The launch's arguments where the hardware left them.  A reference to the
+// by-value parameter would have every lane copy all of it to scratch (2,064
+// bytes) for the tile functions to read back.
+typedef const __attribute__((address_space(4))) MultiArgs* KernelArgs;
+
 // Tile t of one shape.  One tile per call and per block: a loop over tiles,
 // in here or around the call, keeps state live across fit_one and costs
-// registers (the kernel would drop to one wave per SIMD).
+// registers (the kernel would drop to one wave per SIMD).  args: the address of
+// the model's FitArgs, made uniform again, so that its values are scalar loads.
 template <int MODEL, int CAM, int N, int L>
-__device__ __attribute__((noinline)) void multi_tile(const FitArgs& a, int32_t first, int32_t count, int32_t t) {
+__device__ __attribute__((noinline)) void multi_tile(uint64_t args, int32_t first, int32_t count, int32_t t) {
   constexpr int RPT = kWave / L;   // ROIs per tile
+  const uint64_t at = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(args >> 32)) << 32 |
+                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)args);
+  FitArgs a;
+  __builtin_memcpy(&a, (const FitArgs*)(const __attribute__((address_space(4))) FitArgs*)at, sizeof(a));
   const int lane = threadIdx.x;
   const int r = (L == 1) ? 0 : (lane & (L - 1));
   // An entry whose first slot is empty holds no ROI of this shape.
@@ -103,27 +113,28 @@ __device__ __attribute__((noinline)) void multi_tile(const FitArgs& a, int32_t f
 }
 
 template <int CAM, int MODEL, int N>
-__device__ __forceinline__ void multi_case(const MultiArgs& m, int q, int t) {
-  const int L = m.lanes[q];
+__device__ __forceinline__ void multi_case(KernelArgs m, int q, int t) {
+  const int L = m->lanes[q];
+  const uint64_t a = (uint64_t)&m->fa[MODEL];
   if constexpr (multi_has(MODEL, CAM, N, 1)) {
-    if (L == 1) { multi_tile<MODEL, CAM, N, 1>(m.fa[MODEL], m.first[q], m.count[q], t); return; }
+    if (L == 1) { multi_tile<MODEL, CAM, N, 1>(a, m->first[q], m->count[q], t); return; }
   }
   if constexpr (multi_has(MODEL, CAM, N, 2)) {
-    if (L == 2) { multi_tile<MODEL, CAM, N, 2>(m.fa[MODEL], m.first[q], m.count[q], t); return; }
+    if (L == 2) { multi_tile<MODEL, CAM, N, 2>(a, m->first[q], m->count[q], t); return; }
   }
   if constexpr (multi_has(MODEL, CAM, N, 8)) {
-    if (L == 8) { multi_tile<MODEL, CAM, N, 8>(m.fa[MODEL], m.first[q], m.count[q], t); return; }
+    if (L == 8) { multi_tile<MODEL, CAM, N, 8>(a, m->first[q], m->count[q], t); return; }
   }
   if constexpr (multi_has(MODEL, CAM, N, 16)) {
-    if (L == 16) { multi_tile<MODEL, CAM, N, 16>(m.fa[MODEL], m.first[q], m.count[q], t); return; }
+    if (L == 16) { multi_tile<MODEL, CAM, N, 16>(a, m->first[q], m->count[q], t); return; }
   }
   if constexpr (multi_has(MODEL, CAM, N, 4)) {
-    if (L == 4) multi_tile<MODEL, CAM, N, 4>(m.fa[MODEL], m.first[q], m.count[q], t);
+    if (L == 4) multi_tile<MODEL, CAM, N, 4>(a, m->first[q], m->count[q], t);
   }
 }
 
 template <int CAM, int MODEL>
-__device__ __forceinline__ void multi_box(const MultiArgs& m, int box, int q, int t) {
+__device__ __forceinline__ void multi_box(KernelArgs m, int box, int q, int t) {
   switch (box) {
     case 3: multi_case<CAM, MODEL, 3>(m, q, t); break;
     case 4: multi_case<CAM, MODEL, 4>(m, q, t); break;
@@ -143,16 +154,19 @@ __device__ __forceinline__ void multi_box(const MultiArgs& m, int box, int q, in
   }
 }
 
-// One block (one wave) per tile; tiles of the heaviest shapes come first.
+// One block (one wave) per tile; tiles of the heaviest shapes come first.  Two
+// waves per SIMD, which binds the tile functions too: left alone, the largest
+// ones take AGPRs beside their 248 VGPRs and the kernel one wave.
 template <int CAM>
-__global__ __launch_bounds__(kWave) void multi_fit(MultiArgs m) {
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void multi_fit(MultiArgs) {
+  const KernelArgs m = (KernelArgs)__builtin_amdgcn_kernarg_segment_ptr();
   const int32_t blk = blockIdx.x;
-  if (blk >= m.block_start[m.n_entries]) return;
+  if (blk >= m->block_start[m->n_entries]) return;
   int q = 0;
-  while (q + 1 < m.n_entries && m.block_start[q + 1] <= blk) ++q;
-  const int s = m.shape[q];
+  while (q + 1 < m->n_entries && m->block_start[q + 1] <= blk) ++q;
+  const int s = m->shape[q];
   const int model = s / kNumBoxes, box = kMinBox + s % kNumBoxes;
-  const int tt = blk - m.block_start[q];
+  const int tt = blk - m->block_start[q];
   switch (model) {
     case XYNB: multi_box<CAM, XYNB>(m, box, q, tt); break;
     case XYNBS: multi_box<CAM, XYNBS>(m, box, q, tt); break;
