@@ -33,13 +33,14 @@ __host__ __device__ constexpr bool lanes_built(int box, int lanes) {
   return (lanes == 1 && box <= 12) || lanes == 2 || lanes == 4 || lanes == 8 || lanes == 16;
 }
 
-// Largest box size whose kernel with `lanes` lanes per ROI still fits 256
-// VGPRs without spilling, i.e. runs two or more waves per SIMD, with a few
-// registers to spare for the multi-shape kernel's call.  A lane keeps its
-// ceil(box / lanes) pixel columns (and, for sCMOS, their variances) in VGPRs
-// for the whole fit.  From the gfx950 build's register counts
-// (kernel-resource-usage): 4 lanes fit every box except astigmatic sCMOS ROIs
-// of 14 px and up, 8 lanes every box but 16 px outside XYNB, 16 lanes all.
+// Largest box size whose tile with `lanes` lanes per ROI the multi-shape kernels
+// hold (gmle_multi.hpp): together they have to stay within 256 VGPRs, two waves
+// per SIMD (248 in this build, both cameras).  A lane keeps its
+// ceil(box / lanes) pixel columns (and, for sCMOS, their variances) in VGPRs for
+// the whole fit.  The lines were drawn for kernels that held more registers; all
+// tiles within them still fit.  One more box on one lane (sCMOS 6-7 px, ideal 8 px
+// with a width) fits too, but the mode's lanes do not depend on the batch's size,
+// and 2,000 ROIs of sCMOS XYNB 7 px took 71 us on one lane and 51 on two.
 __host__ __device__ constexpr int max_box_within_256(int model, int camera, int lanes) {
   const bool sc = camera == SCMOS;
   if (lanes == 1)
@@ -53,10 +54,12 @@ __host__ __device__ constexpr int max_box_within_256(int model, int camera, int 
   return kMaxSmallBox;
 }
 
-// Lanes per ROI of a large box (above kMaxSmallBox) in a large batch: 8 where
-// that kernel fits 256 VGPRs (two waves per SIMD), else 16.  From the gfx950
-// build's register counts: 8 lanes fit up to 24 px (216-256 VGPRs) except
-// astigmatic sCMOS ROIs above 20 px; 16 lanes fit up to 32 px (161-245).
+// Lanes per ROI of a large box (above kMaxSmallBox) in a large batch: 8, whose
+// waves repeat less per-ROI work than 16.  100,000 ROIs, us per launch on 8 and 16
+// lanes: XYNB 17 px 366 / 450, XYNBS 21 px 535 / 777, XYNBSXSY 24 px sCMOS 660 / 969.
+// 16 above 24 px, where 8 are not built, and for astigmatic sCMOS ROIs above
+// 20 px: a line drawn for kernels that held more registers, and part of what
+// gmle_default_lanes promises (24 px now 716 / 994).
 __host__ __device__ constexpr int large_box_lanes(int model, int camera, int box) {
   return (box <= 24 && !(model == ASTIG && camera == SCMOS && box > 20)) ? 8 : 16;
 }

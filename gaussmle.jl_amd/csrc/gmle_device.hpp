@@ -27,11 +27,10 @@ constexpr int kDppSwap2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141;  // row_half_mirror
 constexpr int kDppMirror = 0x140;      // row_mirror
 
-// bound_ctrl is set: a lane whose source falls outside its row reads 0
-// instead of an undefined value.  Only row_shr in group_next<8> has such lanes,
-// and their values are never selected.  With it set, the compiler folds the
-// move into the add or subtraction that reads it (v_add_f32_dpp): one VALU
-// instruction fewer per reduction step.
+// bound_ctrl is set: a lane whose source falls outside its row would read 0 (no
+// move here has one).  With it set, the compiler folds the move into the add or
+// subtraction that reads it (v_add_f32_dpp): one VALU instruction fewer per
+// reduction step.
 template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
@@ -67,29 +66,11 @@ template <int L> __device__ __forceinline__ float group_max(float v) {
   return v;
 }
 
-// Moves inside a group of L lanes (lane r of a group is lane r of its ROI):
-//   group_next<L>(v):     lane r receives lane (r + 1) mod L's v
-//   group_bcast<L, O>(v): every lane receives lane O's v
-// quad_perm patterns for 2 and 4 lanes, row_ror / row_newbcast for 16 (one
-// DPP row), and two row moves plus a select for the half rows of 8.
-constexpr int kDppRowShr = 0x110;       // row_shr:n = 0x110 + n, lane i <- i - n
-constexpr int kDppRowRor = 0x120;       // row_ror:n = 0x120 + n, lane i <- (i - n) mod 16
+// Inside a group of L lanes (lane r of a group is lane r of its ROI),
+// group_bcast<L, O>(v): every lane receives lane O's v.  quad_perm patterns for
+// 2 and 4 lanes, row_newbcast for 16 (one DPP row), and two of them plus a select
+// for the half rows of 8.
 constexpr int kDppRowNewBcast = 0x150;  // row_newbcast:n = 0x150 + n, lane i <- lane n of its row
-
-template <int L> __device__ __forceinline__ float group_next(float v) {
-  static_assert(L == 2 || L == 4 || L == 8 || L == 16, "groups of 2, 4, 8 or 16 lanes");
-  if constexpr (L == 2) {
-    return dpp_move<kDppSwap1>(v);
-  } else if constexpr (L == 4) {
-    return dpp_move<0x39>(v);   // quad_perm [1,2,3,0]
-  } else if constexpr (L == 16) {
-    return dpp_move<kDppRowRor + 15>(v);
-  } else {
-    const float a = dpp_move<kDppRowRor + 15>(v);   // lane i <- (i + 1) mod 16
-    const float b = dpp_move<kDppRowShr + 7>(v);    // lanes 7 and 15 <- lanes 0 and 8
-    return (threadIdx.x & 7) == 7 ? b : a;
-  }
-}
 
 template <int L, int O> __device__ __forceinline__ float group_bcast(float v) {
   static_assert(L == 2 || L == 4 || L == 8 || L == 16, "groups of 2, 4, 8 or 16 lanes");
@@ -121,9 +102,6 @@ __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcp
 // min / max propagate NaN.
 template <class T> __device__ __forceinline__ T jclamp(T x, T lo, T hi) {
   return x > hi ? hi : (x < lo ? lo : x);
-}
-template <class T> __device__ __forceinline__ T jmin(T x, T y) {
-  return (x != x || y != y) ? (x + y) : (y < x ? y : x);
 }
 template <class T> __device__ __forceinline__ T jmax(T x, T y) {
   return (x != x || y != y) ? (x + y) : (y > x ? y : x);

@@ -68,7 +68,6 @@ template <class T> struct DM;
 template <> struct DM<float> {
   // Axis scales carry sqrt(log2 e): t * s is v = k u of gmle_erf.hpp, so the
   // Gaussian exp(-u^2) is exp2(-v^2).
-  static __device__ __forceinline__ float erf_scale() { return kErfK; }
   // exp(-u^2), and the edge's signed erfc and half-sign for the pixel
   // integrals (gmle_erf.hpp), which reuse the Gaussian
   static __device__ __forceinline__ void erf_gauss(float t, float s, float& se, float& hs, float& g) {
@@ -79,7 +78,6 @@ template <> struct DM<float> {
   static __device__ __forceinline__ float inv_sqrt_2pi() { return kInvSqrt2Pi; }
   // a / b for the per-iteration width and axis constants: one v_rcp_f32
   // (1 ulp) and a multiply instead of the ~10-instruction IEEE division.
-  // The Newton step keeps the IEEE division.
   static __device__ __forceinline__ float div(float a, float b) { return a * fast_rcp(b); }
   // 1 / b: v_rcp_f32 and one Newton step (correctly rounded but for rare last
   // bits), left out where the reciprocal is not finite.
@@ -94,7 +92,6 @@ template <> struct DM<float> {
   static __device__ __forceinline__ float erf_rate(float, float inv_s) { return fabsf(inv_s) * kErfRate; }
 };
 template <> struct DM<double> {
-  static __device__ __forceinline__ double erf_scale() { return 1.0; }
   // Float64 keeps the reference's erf difference: its cancellation (~1e-16
   // absolute) is negligible, and tails that erf rounds to exactly +-1 stay
   // exactly 0 as in the reference.  se = -erf(u), hs = 0 in pixel_integral.
@@ -131,7 +128,8 @@ template <class T, int M> struct AxisTab {
 template <class T, int M, bool SIG>
 __device__ __forceinline__ void axis_tables(T mu, T sigma, T nph, int first, AxisTab<T, M>& tb) {
   const T inv_s = DM<T>::div(T(1), sigma);
-  const T s_erf = sqrt(DM<T>::div(T(0.5), sigma * sigma)) * DM<T>::erf_scale();
+  static_assert(sizeof(T) == 8, "the Float32 edges are scaled (erf_rate)");
+  const T s_erf = sqrt(DM<T>::div(T(0.5), sigma * sigma));
   const T c = -nph * DM<T>::inv_sqrt_2pi() * inv_s;
   const T c2 = c * inv_s * inv_s;
   const T cs = c * inv_s;
@@ -367,9 +365,9 @@ template <int N, int L> constexpr int block_cols() {
 template <int CB> constexpr int rows_together() { return CB == 1 ? 2 : 1; }
 // Least waves per SIMD a fit kernel is built for: three where a lane's pixels (and
 // variances) leave the loop enough of the 168 VGPRs that three waves have, and
-// three waves' LDS fits a CU's 160 KB, else two where a few spilled values
-// reach them (sCMOS XYNBS 16 px on 4 lanes, 128 values, needs 258 VGPRs: 4.19
-// against 2.93 ms per 1M ROIs at one wave and two).  Above the first line the
+// three waves' LDS fits a CU's 160 KB, else two up to 144 values (sCMOS XYNBS
+// 16 px on 4 lanes, 128 values: 235 VGPRs; at one wave an earlier build of it took
+// 4.19 ms per 1M ROIs, at two 2.93).  Above the first line the
 // spills cost more than the third wave hides: sCMOS XYNBS 13 px
 // on 4 lanes (86 values) runs 2.46 -> 2.34 ms per 1M ROIs with three waves and
 // 164 B of scratch, XYNB 11 px on one lane (121 values) 1.51 -> 2.04 ms.
@@ -767,18 +765,10 @@ __device__ __forceinline__ void gradient(const PixelSums& u, const AxisK<float>&
 // kernel) or global memory (GlobalSrc, in the Float64 final-pass kernel).
 // ---------------------------------------------------------------------------
 template <int N, bool SC> struct RegSrc {
-  static constexpr bool kInRegisters = true;
   const float* dv;   // this lane's column block, [cc * N + i]
   const float* vr;
   __device__ __forceinline__ float d(int cc, int i) const { return dv[cc * N + i]; }
   __device__ __forceinline__ float var(int cc, int i) const { return SC ? vr[cc * N + i] : 0.f; }
-  __device__ __forceinline__ void column(int cc, float* dcol, float* vcol) const {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      dcol[i] = dv[cc * N + i];
-      if constexpr (SC) vcol[i] = vr[cc * N + i];
-    }
-  }
 };
 // n consecutive floats from p (4-byte aligned) in 16- and 8-byte loads: gfx950
 // global loads need only dword alignment, and one lane's run of a column then
@@ -804,25 +794,15 @@ template <int n> __device__ __forceinline__ void load_run(const float* p, float*
 }
 
 template <int N, bool SC> struct GlobalSrc {
-  static constexpr bool kInRegisters = false;
   const float* data = nullptr;   // the ROI, column-major
   const float* var = nullptr;    // var_map at the ROI's first pixel
   int ny = 0;
-  __device__ __forceinline__ float d(int cc, int i) const { return data[cc * N + i]; }
-  __device__ __forceinline__ float var_at(int cc, int i) const { return var[(int64_t)cc * ny + i]; }
   // column cc's pixels and variances (both runs are contiguous)
   __device__ __forceinline__ void column(int cc, float* dcol, float* vcol) const {
     load_run<N>(data + cc * N, dcol);
     if constexpr (SC) load_run<N>(var + (int64_t)cc * ny, vcol);
   }
 };
-template <int N, bool SC> __device__ __forceinline__ float src_var(const RegSrc<N, SC>& s, int cc, int i) {
-  return s.var(cc, i);
-}
-template <int N, bool SC> __device__ __forceinline__ float src_var(const GlobalSrc<N, SC>& s, int cc, int i) {
-  return s.var_at(cc, i);
-}
-
 template <class TF, int P> struct FinalOut {
   TF crlb[P];
   TF llr;
@@ -834,27 +814,15 @@ template <class TF, int P> struct FinalOut {
 // upper triangle Fu.  du holds the pixel's P model derivatives.
 template <int CAM, int P, class TF>
 __device__ __forceinline__ void final_pixel(TF d, TF var, TF mu, const TF* du, bool cvalid, TF* Fu, TF& llr) {
-  constexpr bool F32 = sizeof(TF) == 4;
+  static_assert(sizeof(TF) == 8, "the Float32 pass sums its Fisher matrix by columns and rows");
   TF v = mu;
   TF lp;
   TF rv = TF(0);   // 1/mu, the ideal camera's Fisher weight
   if constexpr (CAM == IDEAL) {
     // camera_models.jl:60-71, as d log(mu/d) + d - mu with one log:
     // d log(mu/d) = -d log(d (1/mu)), and 1/mu is also the Fisher weight below.
-    // Float32 takes 1/mu from v_rcp_f32 (1 ulp); the single log also avoids
-    // the cancellation of d log(mu) against d log(d) in the two-log form.
-    if constexpr (F32) {
-      // ln x as v_log_f32 (log2) times ln 2.  x = d/mu of a pixel with d > 0
-      // lies far above the denormal range; the clamp keeps even a denormal
-      // product finite (its term is then ~0, as it would be).
-      rv = mu > TF(0) ? fast_rcp(mu) : TF(0);
-      const float x = fmaxf(d * rv, 1.17549435e-38f);
-      const float lnx = __builtin_amdgcn_logf(x) * 0.693147180559945309f;
-      lp = (mu > TF(0) && d > TF(0)) ? -d * lnx + (d - mu) : (mu > TF(0) && d == TF(0)) ? -mu : TF(0);
-    } else {
-      rv = mu > TF(0) ? TF(1) / mu : TF(0);
-      lp = (mu > TF(0) && d > TF(0)) ? -d * log(d * rv) + (d - mu) : (mu > TF(0) && d == TF(0)) ? -mu : TF(0);
-    }
+    rv = mu > TF(0) ? TF(1) / mu : TF(0);
+    lp = (mu > TF(0) && d > TF(0)) ? -d * log(d * rv) + (d - mu) : (mu > TF(0) && d == TF(0)) ? -mu : TF(0);
   } else {
     // camera_models.jl:73-85.  The Fisher weight below divides again, inside
     // its own block: a 1/v shared by both keeps it live across the block, and
@@ -959,16 +927,9 @@ __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass(const float* th
       final_pixel<CAM, P, TF>((TF)dcol[i], CAM == SCMOS ? (TF)vcol[i] : TF(0), mu, du, cvalid, Fu, llr);
     }
   };
-  if constexpr (Src::kInRegisters) {
-    // VGPR-resident pixels: the column index must be a compile-time constant.
-#pragma unroll
-    for (int cc = 0; cc < CB; ++cc) column(cc);
-  } else {
-    // Pixels from memory: one column at a time keeps only that column's loads
-    // in flight.
+  // One column at a time keeps only that column's loads in flight.
 #pragma unroll 1
-    for (int cc = 0; cc < CB; ++cc) column(cc);
-  }
+  for (int cc = 0; cc < CB; ++cc) column(cc);
   return final_reduce<L, P, TF>(Fu, llr);
 }
 
@@ -979,7 +940,6 @@ __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass(const float* th
 template <int MODEL, int CAM, int N, int L, class TF, class Src>
 __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass_rows(const float* th, const float* psf, int c0,
                                                                     const Src& src) {
-  static_assert(Src::kInRegisters, "rows outer needs register-resident pixels");
   using Tr = MT<MODEL>;
   constexpr int P = Tr::P;
   constexpr int CB = (N + L - 1) / L;
@@ -1032,32 +992,26 @@ __device__ __forceinline__ FinalOut<TF, MT<MODEL>::P> final_pass_rows(const floa
 
 // One pixel's LLR term lp (camera_models.jl:60-85) and Fisher weight wv: 1/v
 // where the model is > 0, else 0 (v = model, or model + variance for sCMOS).
-template <int CAM, class T> __device__ __forceinline__ void final_weights(T d, T var, T mu, T& lp, T& wv) {
-  constexpr bool F32 = sizeof(T) == 4;
+template <int CAM> __device__ __forceinline__ void final_weights(float d, float var, float mu, float& lp, float& wv) {
   if constexpr (CAM == IDEAL) {
     // camera_models.jl:60-71, as d log(mu/d) + d - mu with one log:
     // d log(mu/d) = -d log(d (1/mu)), and 1/mu is also the Fisher weight.
-    // Float32 takes 1/mu from v_rcp_f32 (1 ulp); the single log also avoids
-    // the cancellation of d log(mu) against d log(d) in the two-log form.
-    if constexpr (F32) {
-      // ln x as v_log_f32 (log2) times ln 2.  x = d/mu of a pixel with d > 0
-      // lies far above the denormal range; the clamp keeps even a denormal
-      // product finite (its term is then ~0, as it would be).
-      wv = mu > T(0) ? fast_rcp(mu) : T(0);
-      const float x = fmaxf(d * wv, 1.17549435e-38f);
-      const float lnx = __builtin_amdgcn_logf(x) * 0.693147180559945309f;
-      lp = (mu > T(0) && d >= T(0)) ? -d * lnx + (d - mu) : T(0);   // -mu at d = 0 (lnx is finite there)
-    } else {
-      wv = mu > T(0) ? T(1) / mu : T(0);
-      lp = (mu > T(0) && d > T(0)) ? -d * log(d * wv) + (d - mu) : (mu > T(0) && d == T(0)) ? -mu : T(0);
-    }
+    // 1/mu is v_rcp_f32 (1 ulp); the single log also avoids the cancellation of
+    // d log(mu) against d log(d) in the two-log form.
+    // ln x as v_log_f32 (log2) times ln 2.  x = d/mu of a pixel with d > 0
+    // lies far above the denormal range; the clamp keeps even a denormal
+    // product finite (its term is then ~0, as it would be).
+    wv = mu > 0.f ? fast_rcp(mu) : 0.f;
+    const float x = fmaxf(d * wv, 1.17549435e-38f);
+    const float lnx = __builtin_amdgcn_logf(x) * 0.693147180559945309f;
+    lp = (mu > 0.f && d >= 0.f) ? -d * lnx + (d - mu) : 0.f;   // -mu at d = 0 (lnx is finite there)
   } else {
-    const T v = mu + var;   // camera_models.jl:73-85
-    const T res = d - mu;
-    const T rv = T(1) / v;
+    const float v = mu + var;   // camera_models.jl:73-85
+    const float res = d - mu;
+    const float rv = 1.f / v;
     // the clamp: 1 / v of a denormal v is infinite, and 0 x inf no LLR term
-    lp = v > T(0) ? T(-0.5) * (res * res * fminf(rv, 3.40282347e38f)) : T(0);
-    wv = mu > T(0) ? rv : T(0);
+    lp = v > 0.f ? -0.5f * (res * res * fminf(rv, 3.40282347e38f)) : 0.f;
+    wv = mu > 0.f ? rv : 0.f;
   }
 }
 
@@ -1283,7 +1237,7 @@ __device__ __forceinline__ FinalOut<float, MT<MODEL>::P> final_pass_f32(const fl
       const Band<float> b{v.phi, v.dg, v.w, 0.f};
       const float mu = fmaf(nph * tl.phi, b.phi, bg);
       float lp, wv;
-      final_weights<CAM, float>(dt[s], CAM == SCMOS ? vt[s] : 0.f, mu, lp, wv);
+      final_weights<CAM>(dt[s], CAM == SCMOS ? vt[s] : 0.f, mu, lp, wv);
       if ((L - 1) * RS + s >= N) {
         const bool ok = r * RS + s < N;
         lp = ok ? lp : 0.f;
@@ -1313,7 +1267,7 @@ __device__ __forceinline__ FinalOut<float, MT<MODEL>::P> final_pass_f32(const fl
     for (int cc = 0; cc < CB; ++cc) {
       const float mu = fmaf(cb[cc].phi, pn, bg);
       float lp, wv;
-      final_weights<CAM, float>(dv[cc * N + i], CAM == SCMOS ? vr[cc * N + i] : 0.f, mu, lp, wv);
+      final_weights<CAM>(dv[cc * N + i], CAM == SCMOS ? vr[cc * N + i] : 0.f, mu, lp, wv);
       if (may_pad<N, L>(cc)) {
         lp = c0 + cc < N ? lp : 0.f;
         wv = c0 + cc < N ? wv : 0.f;
