@@ -350,11 +350,12 @@ def run_boxer(n_frames: int = 32, reps: int = 10, cpu: bool = True) -> dict:
     n = int(out["count"].item())
     npix = ny * nx * n_frames
     win = gbx.suppression_radius(c["boxsize"], c["overlap"])
-    # algorithmic HBM bytes: frames read, filtered stack written, candidate /
-    # survivor words (8 B per 64 pixels, written and read twice), each
-    # detection's window re-read and its box read and written
-    per_pix = 4 + 4 + 4 * 8 / 64
-    per_det = (2 * win + 1) ** 2 * 4 + 2 * c["boxsize"] ** 2 * 4 + 16
+    # algorithmic HBM bytes: frames read, candidate and survivor words (8 B per
+    # 60 rows of a column, each written and read), and per detection its window
+    # of the filtered stack, which is stored around bright pixels only, written
+    # and read, and its box read and written
+    per_pix = 4 + 4 * 8 / 60
+    per_det = 2 * (2 * win + 1) ** 2 * 4 + 2 * c["boxsize"] ** 2 * 4 + 16
     algo = per_pix * npix + per_det * n
     res = {"frames": n_frames, "frame_shape": [ny, nx], "detections": n, "ms_per_call": round(t * 1e3, 4),
            "frames_per_s": round(n_frames / t, 1), "pixels_per_s": round(npix / t, 1),
