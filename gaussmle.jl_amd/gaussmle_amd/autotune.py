@@ -10,7 +10,8 @@ batch also on what runs beside it.  The tuner:
   2. refines in the batch itself: coordinate descent over the shapes, timing
      the whole batched call, keeping a change only when it is faster;
   3. picks the number of streams the per-shape launches are spread over, or
-     the one-launch mode (every shape in one multi-shape kernel, 4 lanes).
+     the one-launch mode (every shape in one multi-shape kernel, on the table's
+     lanes where that kernel has the tile, else 4).
 All timings are HIP-event times on the device, median of `reps` runs.
 """
 from __future__ import annotations
@@ -142,7 +143,7 @@ def tune(mb: gb.MixedBatch, d: dict, precision: str = "fp32", reps: int = 3, sta
         if t < cur * 0.99:
             tuning.streams, cur = s, t
     if precision == "fp32":
-        # one launch for every shape (4 lanes per ROI; the lanes table is unused)
+        # one launch for every shape
         t = batch_ms(tuning.lanes, 0)
         tuning.history.append(("one_launch", t))
         tuning.one_launch_ms = t
