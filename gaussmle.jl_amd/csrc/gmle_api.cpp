@@ -127,8 +127,10 @@ int one_launch_lanes(int model, int camera, int box, int lanes) {
 // the most lanes that keep the launch within one wave per SIMD.  Below that
 // the chip is latency-bound and more, shorter waves finish sooner; above it
 // the extra waves share SIMDs and the replicated per-ROI work costs more than
-// it saves.  Measured on XYNB 11 px and sCMOS XYNBS 13 px: 1K and 4K ROIs run
-// fastest at 16 lanes, 10K at 4, 30K at 2.
+// it saves.  us per launch on 2, 4, 8 and 16 lanes, XYNB 11 px: 1,000 ROIs 60, 38,
+// 32, 22; 10,000 62, 39, 47, 44; 30,000 65, 60, 83, 104.  sCMOS XYNBS 13 px: 1,000
+// 93, 60, 41, 28; 10,000 94, 64, 59, 59; 30,000 97, 104, 108, 139.  So the line is up
+// to 8 % off the best near one wave per SIMD.
 int default_lanes(int model, int camera, int box, int precision, int64_t n_rois) {
   (void)precision;
   const int64_t fill = 256 * 4 * 64;   // CUs x SIMDs x lanes: one wave per SIMD
